@@ -104,6 +104,14 @@ int pi05_prefix_forward(pi05_prefix_ctx* ctx, const void* embeds, const uint8_t*
                         void* const* k_layers, void* const* v_layers, int64_t kv_batch_stride,
                         int64_t kv_row_stride, void* stream);
 
+/* One matrix product of the prefill and the vision tower on its own (a parity / debug hook):
+ * C[M, N] = A[M, K] . W[N, K]^T, bf16 operands with rows of lda / ldw elements, on tile `cfg`
+ * (0 .. 7) with epilogue `epi` (0: bf16, optional fp32 bias[N]; 1: the same through GELU; 2: fp32
+ * partial sums of `split` K splits, [split][M][ldc]; 3: GeGLU over W rows that alternate 16 gate and
+ * 16 up rows, bf16 [M, N / 2]).  PI05_E_INVALID, and nothing enqueued, for a product that the tile does not take. */
+int pi05_debug_product(int cfg, int epi, const void* a, const void* w, void* c, const float* bias, int M, int N, int K, int lda,
+                       int ldw, int ldc, int split, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

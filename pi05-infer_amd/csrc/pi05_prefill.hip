@@ -2,13 +2,14 @@
 // producing the per-layer K/V cache the denoise loop consumes (_build_prefix_cache,
 // engine.py:770-794).  Layer l (modeling_gemma.py:460-517):
 //   n  = RMSNorm(h)                          rmsnorm_kernel
-//   qkv = n . [Wq; Wk; Wv]^T                 hipBLASLt (bf16 in/out, fp32 accumulation)
+//   qkv = n . [Wq; Wk; Wv]^T                 product (bf16 in/out, fp32 accumulation)
 //   q, k <- RoPE; k, v -> cache              rope_kv_kernel
 //   o  = softmax(q k^T / 16 + mask) v        prefix_attn_kernel (MFMA, K/V staged through LDS)
-//   h += o . Wo^T; n = RMSNorm(h)            hipBLASLt + rmsnorm_kernel (residual fused)
-//   gu = n . [Wg; Wu]^T                      hipBLASLt, N = 32768 in one GEMM
-//   a  = gelu_tanh(g) * u                    geglu_kernel
-//   h += a . Wd^T; n = RMSNorm(h)            hipBLASLt + rmsnorm_kernel
+//   h += o . Wo^T; n = RMSNorm(h)            product (K splits) + rmsnorm_kernel (residual fused)
+//   a  = gelu_tanh(n . Wg^T) * (n . Wu^T)    product, N = 32768, GeGLU in its epilogue
+//   h += a . Wd^T; n = RMSNorm(h)            product (K splits) + rmsnorm_kernel
+// The products run on pi05_mm.h; from kLibRows rows on, q|k|v, o_proj and down_proj on hipBLASLt where it
+// measured faster when the context was created.
 // The last layer computes only its K/V (patches/prefix_last_layer.py:84-112).  Every valid
 // token attends to every valid token of its sample (pi0_pytorch.py:236-250); positions are
 // cumsum(pad) - 1 (engine.py:776).
@@ -22,6 +23,7 @@
 
 #include "pi05_blocks.h"
 #include "pi05_gemm.h"
+#include "pi05_mm.h"
 #include "pi05_prefill.h"
 
 namespace pi05 {
@@ -33,13 +35,18 @@ constexpr int kPHD = kHeads * kHeadDim;      // 2048 attention output columns
 constexpr int kPQkvN = kPHD + 2 * kHeadDim;  // 2560 fused q|k|v columns
 constexpr int kPKvN = 2 * kHeadDim;          // 512: k|v columns (the K/V-only last layer)
 constexpr int kPGuN = 2 * kPI;               // 32768 fused gate|up columns
-// per-layer packed weights (bf16 elements): [q; k; v] | o | [gate; up] | down, nn.Linear layout
+// per-layer packed weights (bf16 elements): [q; k; v] | o | gate and up, 16 rows in turn | down, nn.Linear layout
 constexpr size_t kPOffQkv = 0;
 constexpr size_t kPOffO = kPOffQkv + (size_t)kPQkvN * kPW;
 constexpr size_t kPOffGu = kPOffO + (size_t)kPW * kPHD;
 constexpr size_t kPOffD = kPOffGu + (size_t)kPGuN * kPW;
 constexpr size_t kPLayerElems = kPOffD + (size_t)kPW * kPI;
-constexpr int kDownSplits = 4;  // down_proj / o_proj split-K candidates: 4 slices of K
+// K splits of o_proj and down_proj at most: 8 where few tiles leave CUs idle, 4 beyond kSplitRows rows (the
+// partials grow with the rows: 4 splits hold 32 KiB a row)
+constexpr int kMaxSplits = 8, kSplitRows = 3072;
+int max_splits(int M) { return M <= kSplitRows ? kMaxSplits : 4; }
+// rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate
+constexpr int kLibRows = 1024;
 constexpr int kAttnMtPerWg = 8;  // attention m-tiles (16 query rows: 2 tokens x 8 heads) per workgroup
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt not waited for (gfx9 encoding:
 // vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14])
@@ -92,16 +99,16 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const u16* x, const u16* y
   const u16x8 xv = *reinterpret_cast<const u16x8*>(x + off);
   float h[8];
   if (ys) {
-    float4 a[kDownSplits][2];
+    float4 a[kMaxSplits][2];
 #pragma unroll
-    for (int sp = 0; sp < kDownSplits; ++sp)
+    for (int sp = 0; sp < kMaxSplits; ++sp)
       if (sp < nsplit) {
         const float* q = ys + (size_t)sp * split_stride + off;
         a[sp][0] = *reinterpret_cast<const float4*>(q), a[sp][1] = *reinterpret_cast<const float4*>(q + 4);
       }
     float acc[8] = {a[0][0].x, a[0][0].y, a[0][0].z, a[0][0].w, a[0][1].x, a[0][1].y, a[0][1].z, a[0][1].w};
 #pragma unroll
-    for (int sp = 1; sp < kDownSplits; ++sp)
+    for (int sp = 1; sp < kMaxSplits; ++sp)
       if (sp < nsplit) {
         acc[0] += a[sp][0].x, acc[1] += a[sp][0].y, acc[2] += a[sp][0].z, acc[3] += a[sp][0].w;
         acc[4] += a[sp][1].x, acc[5] += a[sp][1].y, acc[6] += a[sp][1].z, acc[7] += a[sp][1].w;
@@ -380,22 +387,6 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* po, const 
   *reinterpret_cast<u16x8*>(out + ((size_t)b * P + token) * kPHD + head * kHeadDim + d0) = r8;
 }
 
-// ---------------------------------------------------------------------------------------------
-// act = bf16(gelu_tanh(g) * u) over gu rows [g (16384) | u (16384)] (modeling_gemma.py:147 with
-// the fused pointwise rounding: fp32 on the bf16 GEMM outputs, one rounding)
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void geglu_kernel(const u16* gu, u16* act, size_t chunks) {
-  for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < chunks; c += (size_t)gridDim.x * 256) {
-    const size_t row = c / (kPI / 8), j = (c % (kPI / 8)) * 8;
-    const u16x8 gv = *reinterpret_cast<const u16x8*>(gu + row * kPGuN + j);
-    const u16x8 uv = *reinterpret_cast<const u16x8*>(gu + row * kPGuN + kPI + j);
-    u16x8 o;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = f2bf(fmul(gelu_tanh(bf2f(gv[i])), bf2f(uv[i])));
-    *reinterpret_cast<u16x8*>(act + row * kPI + j) = o;
-  }
-}
-
 // out[i] = bf16(table[ids[i]] * sqrt(2048)); an id outside [0, vocab) zero-fills its row and
 // sets *err.
 // A row whose id is outside [0, vocab) is written as zeros and the call's tag goes to a pinned
@@ -425,9 +416,9 @@ struct LayerBind {
 // Device layout of one context: sizes in bytes.
 struct PrefixPlan {
   int L = 0, B = 0, P = 0, M = 0, s_pad = 0, n_mt = 0, items = 0, nsplit = 1;
-  size_t w, ln, h, n, y, qkv, attn, gu, act, qf, kv, pos, valid, invf, rtab, ws, po, pml, dpart;
+  size_t w, ln, h, n, y, qkv, attn, act, qf, kv, pos, valid, invf, rtab, ws, po, pml, dpart;
   size_t total() const {
-    return w + ln + 3 * h + qkv + attn + gu + act + qf + 2 * kv + pos + valid + invf + rtab + ws + po + pml + dpart + 16 * 256;
+    return w + ln + 3 * h + qkv + attn + act + qf + 2 * kv + pos + valid + invf + rtab + ws + po + pml + dpart + 16 * 256;
   }
 };
 constexpr size_t kWorkspace = 64ull << 20;
@@ -453,7 +444,6 @@ PrefixPlan plan_of(const pi05_prefix_dims& d) {
   p.h = rup(M * kPW * 2);
   p.qkv = rup(M * kPQkvN * 2);
   p.attn = rup(M * kPHD * 2);
-  p.gu = rup(M * kPGuN * 2);
   p.act = rup(M * kPI * 2);
   p.qf = rup((size_t)p.B * p.s_pad * kHeads * kHeadDim * 2);
   p.kv = rup((size_t)p.B * p.s_pad * kHeadDim * 2);
@@ -465,7 +455,7 @@ PrefixPlan plan_of(const pi05_prefix_dims& d) {
   const size_t rows = (size_t)p.B * p.n_mt * 16;
   p.po = p.nsplit > 1 ? rup((size_t)p.nsplit * rows * kHeadDim * 4) : 0;
   p.pml = p.nsplit > 1 ? rup((size_t)p.nsplit * rows * 2 * 4) : 0;
-  p.dpart = rup((size_t)kDownSplits * M * kPW * 4);
+  p.dpart = rup((size_t)max_splits(p.M) * M * kPW * 4);
   return p;
 }
 
@@ -514,19 +504,20 @@ struct pi05_prefix_ctx {
   std::vector<LayerBind> binds;
   bool refreshed = false;
   char* base = nullptr;
-  u16 *w = nullptr, *h = nullptr, *n = nullptr, *y = nullptr, *qkv = nullptr, *attn = nullptr, *gu = nullptr, *act = nullptr;
+  u16 *w = nullptr, *h = nullptr, *n = nullptr, *y = nullptr, *qkv = nullptr, *attn = nullptr, *act = nullptr;
   u16 *qf = nullptr, *kf = nullptr, *vf = nullptr;
   float *ln = nullptr, *inv_freq = nullptr, *po = nullptr, *pml = nullptr, *dpart = nullptr;
   u16* rope_tab = nullptr;  // [P + 1][cos | sin] bf16, row = position + 1
-  bool down_split = false;  // down_proj as kDownSplits fp32 split-K GEMMs reduced in the residual norm
-  bool o_split = false;     // o_proj likewise
   int* pos = nullptr;
   uint8_t* valid = nullptr;
   unsigned* host_bad = nullptr;  // pinned host word: tag of the last embed call that met a bad token id
   unsigned embed_tag = 0, reported_tag = 0;
   void* ws = nullptr;
   hipblasLtHandle_t lt = nullptr;
-  GemmPlan g_qkv, g_kv, g_o, g_gu, g_d, g_dsk, g_osk;
+  // the products: on pi05_mm.h, or (from kLibRows rows, where it measured faster) on hipBLASLt
+  GemmPlan g_qkv, g_kv, g_o, g_d;
+  MmPlan m_qkv, m_kv, m_o, m_gu, m_d;
+  bool lib_qkv = false, lib_kv = false, lib_o = false, lib_d = false;
 };
 
 namespace {
@@ -541,16 +532,15 @@ int hip_fail(pi05_prefix_ctx* c, const char* what, hipError_t e) {
   return fail(c, PI05_E_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-GemmOpts split_opts(int ld_k) {
-  GemmOpts o;
-  o.batch = kDownSplits;
-  o.ld_k = ld_k;
-  return o;
-}
-
 int gemm(pi05_prefix_ctx* c, const GemmPlan& p, const u16* W, const u16* A, void* C, hipStream_t st) {
   const hipblasStatus_t s = run_plan(c->lt, p, p.algo, p.ws, W, A, C, nullptr, c->ws, st);
   if (!lt_ok(s)) return fail(c, PI05_E_HIP, "hipblasLtMatmul failed (status " + std::to_string((int)s) + ")");
+  return PI05_OK;
+}
+
+// One product of the layer loop: C[M, N] = A[M, K] . W[N, K]^T with epilogue epi.
+int mm(pi05_prefix_ctx* c, const MmPlan& p, int epi, const u16* W, const u16* A, void* C, int N, int K, int ldc, hipStream_t st) {
+  if (!mm_launch(p.cfg, epi, {A, W, C, nullptr, c->plan.M, N, K, K, K, ldc, p.split}, st)) return fail(c, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
 
@@ -624,7 +614,6 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
   c->y = reinterpret_cast<u16*>(take(p.h));
   c->qkv = reinterpret_cast<u16*>(take(p.qkv));
   c->attn = reinterpret_cast<u16*>(take(p.attn));
-  c->gu = reinterpret_cast<u16*>(take(p.gu));
   c->act = reinterpret_cast<u16*>(take(p.act));
   c->qf = reinterpret_cast<u16*>(take(p.qf));
   c->kf = reinterpret_cast<u16*>(take(p.kv));
@@ -658,35 +647,48 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
   }
   std::string perr;
   const int M = p.M;
-  if (!lt_ok(hipblasLtCreate(&c->lt)) || !make_plan(c->lt, M, kPQkvN, kPW, kWorkspace, &c->g_qkv, &perr) ||
-      !make_plan(c->lt, M, kPKvN, kPW, kWorkspace, &c->g_kv, &perr) || !make_plan(c->lt, M, kPW, kPHD, kWorkspace, &c->g_o, &perr) ||
-      !make_plan(c->lt, M, kPGuN, kPW, kWorkspace, &c->g_gu, &perr) || !make_plan(c->lt, M, kPW, kPI, kWorkspace, &c->g_d, &perr) ||
-      !make_plan(c->lt, M, kPW, kPI / kDownSplits, kWorkspace, &c->g_dsk, &perr, split_opts(kPI)) ||
-      !make_plan(c->lt, M, kPW, kPHD / kDownSplits, kWorkspace, &c->g_osk, &perr, split_opts(kPHD))) {
+  const bool lib = M > kLibRows;
+  if (lib && (!lt_ok(hipblasLtCreate(&c->lt)) || !make_plan(c->lt, M, kPQkvN, kPW, kWorkspace, &c->g_qkv, &perr) ||
+              !make_plan(c->lt, M, kPKvN, kPW, kWorkspace, &c->g_kv, &perr) || !make_plan(c->lt, M, kPW, kPHD, kWorkspace, &c->g_o, &perr) ||
+              !make_plan(c->lt, M, kPW, kPI, kWorkspace, &c->g_d, &perr))) {
     if (perr.empty()) perr = "hipblasLtCreate failed";
     pi05_prefix_destroy(c);
     return fail(nullptr, PI05_E_HIP, perr);
   }
-  // pick each GEMM's fastest algorithm on this device and shape
+  // pick each product's fastest tile and split (or hipBLASLt algorithm) on this device and shape
   // (weights rotate over the layers' blocks while timing, as the layer loop streams them)
   const size_t ls = kPLayerElems * 2;
   const int nl = dims->depth;
-  const bool tuned = tune_plan(c->lt, &c->g_qkv, c->w, c->n, c->qkv, c->ws, nullptr, nullptr, ls, nl) &&
-                     tune_plan(c->lt, &c->g_kv, c->w, c->n, c->qkv, c->ws, nullptr, nullptr, ls, nl) &&
-                     tune_plan(c->lt, &c->g_o, c->w, c->attn, c->y, c->ws, nullptr, nullptr, ls, nl) &&
-                     tune_plan(c->lt, &c->g_gu, c->w, c->n, c->gu, c->ws, nullptr, nullptr, ls, nl) &&
-                     tune_plan(c->lt, &c->g_d, c->w, c->act, c->y, c->ws, nullptr, nullptr, ls, nl) &&
-                     tune_plan(c->lt, &c->g_dsk, c->w, c->act, c->dpart, c->ws, nullptr, nullptr, ls, nl) &&
-                     tune_plan(c->lt, &c->g_osk, c->w, c->attn, c->dpart, c->ws, nullptr, nullptr, ls, nl);
+  // what rmsnorm_kernel pays per split: 4 bytes per output element at ~4 TB/s, less the bf16 output
+  // that it would read and the product write otherwise
+  const float part_ms = (float)(4.0 * M * kPW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kPW / 4e12 * 1e3);
+  auto tune_n = [&](const u16* A, int K, MmPlan* o) {  // o_proj, down_proj: one product, or fp32 K splits
+    MmPlan one, sp;
+    if (!mm_tune({A, c->w, c->y, nullptr, M, kPW, K, K, K, kPW, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &one) ||
+        !mm_tune({A, c->w, c->dpart, nullptr, M, kPW, K, K, K, kPW, 1}, kMmF32, 2, max_splits(M), part_ms, ls, nl, nullptr, &sp))
+      return false;
+    *o = sp.ms + part_ms * (float)sp.split - bf_ms < one.ms ? sp : one;
+    return true;
+  };
+  bool tuned = mm_tune({c->n, c->w, c->qkv, nullptr, M, kPQkvN, kPW, kPW, kPW, kPQkvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+               mm_tune({c->n, c->w, c->qkv, nullptr, M, kPKvN, kPW, kPW, kPW, kPKvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_kv) &&
+               mm_tune({c->n, c->w, c->act, nullptr, M, kPGuN, kPW, kPW, kPW, kPI, 1}, kMmGeglu, 1, 1, 0.f, ls, nl, nullptr, &c->m_gu) &&
+               tune_n(c->attn, kPHD, &c->m_o) && tune_n(c->act, kPI, &c->m_d);
+  if (tuned && lib) {
+    tuned = tune_plan(c->lt, &c->g_qkv, c->w, c->n, c->qkv, c->ws, nullptr, nullptr, ls, nl) &&
+            tune_plan(c->lt, &c->g_kv, c->w, c->n, c->qkv, c->ws, nullptr, nullptr, ls, nl) &&
+            tune_plan(c->lt, &c->g_o, c->w, c->attn, c->y, c->ws, nullptr, nullptr, ls, nl) &&
+            tune_plan(c->lt, &c->g_d, c->w, c->act, c->y, c->ws, nullptr, nullptr, ls, nl);
+    auto cost = [&](const MmPlan& m) { return m.split > 1 ? m.ms + part_ms * (float)m.split - bf_ms : m.ms; };
+    c->lib_qkv = c->g_qkv.ms < c->m_qkv.ms;
+    c->lib_kv = c->g_kv.ms < c->m_kv.ms;
+    c->lib_o = c->g_o.ms < cost(c->m_o);
+    c->lib_d = c->g_d.ms < cost(c->m_d);
+  }
   if (!tuned) {
     pi05_prefix_destroy(c);
-    return fail(nullptr, PI05_E_HIP, "GEMM algorithm tuning failed");
+    return fail(nullptr, PI05_E_HIP, "GEMM tuning failed");
   }
-  // split-K down_proj when its GEMM plus the extra partial traffic of the fused reduction
-  // ((kDownSplits * 4 - 2) bytes per output element at ~4 TB/s) beats the single bf16 GEMM
-  const float extra_ms = (float)((double)(kDownSplits * 4 - 2) * M * kPW / 4e12 * 1e3);
-  c->down_split = c->g_dsk.ms + extra_ms < c->g_d.ms;
-  c->o_split = c->g_osk.ms + extra_ms < c->g_o.ms;
   *out = c;
   return PI05_OK;
 }
@@ -696,10 +698,7 @@ int pi05_prefix_destroy(pi05_prefix_ctx* c) {
   free_plan(&c->g_qkv);
   free_plan(&c->g_kv);
   free_plan(&c->g_o);
-  free_plan(&c->g_gu);
   free_plan(&c->g_d);
-  free_plan(&c->g_dsk);
-  free_plan(&c->g_osk);
   if (c->lt) hipblasLtDestroy(c->lt);
   // an embed kernel still in flight may write the pinned word
   if (c->host_bad) {
@@ -734,13 +733,14 @@ int pi05_prefix_refresh_weights(pi05_prefix_ctx* c, void* stream) {
   for (int l = 0; l < c->d.depth; ++l) {
     const LayerBind& b = c->binds[l];
     u16* w = c->w + (size_t)l * kPLayerElems;
-    const size_t sq = (size_t)kPHD * kPW * 2, sk = (size_t)kHeadDim * kPW * 2, sg = (size_t)kPI * kPW * 2;
+    const size_t sq = (size_t)kPHD * kPW * 2, sk = (size_t)kHeadDim * kPW * 2;
     hipError_t e = hipMemcpyAsync(w + kPOffQkv, b.wq, sq, k, st);
     if (e == hipSuccess) e = hipMemcpyAsync(w + kPOffQkv + (size_t)kPHD * kPW, b.wk, sk, k, st);
     if (e == hipSuccess) e = hipMemcpyAsync(w + kPOffQkv + (size_t)(kPHD + kHeadDim) * kPW, b.wv, sk, k, st);
     if (e == hipSuccess) e = hipMemcpyAsync(w + kPOffO, b.wo, (size_t)kPW * kPHD * 2, k, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(w + kPOffGu, b.wg, sg, k, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(w + kPOffGu + (size_t)kPI * kPW, b.wu, sg, k, st);
+    const size_t s16 = (size_t)16 * kPW * 2;  // 16 gate rows, then the same 16 up rows
+    if (e == hipSuccess) e = hipMemcpy2DAsync(w + kPOffGu, 2 * s16, b.wg, s16, s16, kPI / 16, k, st);
+    if (e == hipSuccess) e = hipMemcpy2DAsync(w + kPOffGu + (size_t)16 * kPW, 2 * s16, b.wu, s16, s16, kPI / 16, k, st);
     if (e == hipSuccess) e = hipMemcpyAsync(w + kPOffD, b.wd, (size_t)kPW * kPI * 2, k, st);
     if (e == hipSuccess) e = hipMemcpyAsync(c->ln + (size_t)l * 2 * kPW, b.ln1, kPW * 4, k, st);
     if (e == hipSuccess) e = hipMemcpyAsync(c->ln + (size_t)l * 2 * kPW + kPW, b.ln2, kPW * 4, k, st);
@@ -804,41 +804,45 @@ int pi05_prefix_forward(pi05_prefix_ctx* c, const void* embeds, const uint8_t* p
   const float eps = c->d.rms_eps;
   positions_kernel<<<p.B, 256, 0, st>>>(prefix_pad, p.P, p.s_pad, c->pos, c->valid);
   rmsnorm_kernel<<<p.M, 256, 0, st>>>(emb, nullptr, c->ln, nullptr, c->n, eps);
+  // c->h = x + A . W^T, c->n = RMSNorm(c->h) with weight nw (NULL: the last layer's, which nothing reads)
+  auto residual = [&](bool lib, const GemmPlan& g, const MmPlan& m, const u16* W, const u16* A, int K, const u16* x, const float* nw) {
+    const bool parts = !lib && m.split > 1;
+    const int e = lib ? gemm(c, g, W, A, c->y, st) : mm(c, m, parts ? kMmF32 : kMmBf16, W, A, parts ? (void*)c->dpart : (void*)c->y, kPW, K, kPW, st);
+    if (e != PI05_OK || !nw) return e;
+    if (parts) rmsnorm_kernel<<<p.M, 256, 0, st>>>(x, nullptr, nw, c->h, c->n, eps, c->dpart, m.split, (size_t)p.M * kPW);
+    else rmsnorm_kernel<<<p.M, 256, 0, st>>>(x, c->y, nw, c->h, c->n, eps);
+    return (int)PI05_OK;
+  };
   for (int l = 0; l < p.L; ++l) {
     const u16* w = c->w + (size_t)l * kPLayerElems;
     const float* ln = c->ln + (size_t)l * 2 * kPW;
     const bool kv_only = c->d.skip_last_layer && l == p.L - 1;
     RopeKvArgs ra{c->qkv, kv_only ? kPKvN : kPQkvN, kv_only ? 1 : 0, p.P, p.s_pad, c->pos, c->rope_tab,
                   c->qf, c->kf, c->vf, static_cast<u16*>(k_layers[l]), static_cast<u16*>(v_layers[l]), kv_batch_stride, kv_row_stride};
-    int rc = kv_only ? gemm(c, c->g_kv, w + kPOffQkv + (size_t)kPHD * kPW, c->n, c->qkv, st) : gemm(c, c->g_qkv, w + kPOffQkv, c->n, c->qkv, st);
+    const u16* wkv = w + kPOffQkv + (size_t)kPHD * kPW;
+    int rc;
+    if (kv_only) rc = c->lib_kv ? gemm(c, c->g_kv, wkv, c->n, c->qkv, st) : mm(c, c->m_kv, kMmBf16, wkv, c->n, c->qkv, kPKvN, kPW, kPKvN, st);
+    else rc = c->lib_qkv ? gemm(c, c->g_qkv, w + kPOffQkv, c->n, c->qkv, st) : mm(c, c->m_qkv, kMmBf16, w + kPOffQkv, c->n, c->qkv, kPQkvN, kPW, kPQkvN, st);
     if (rc != PI05_OK) return rc;
     rope_kv_kernel<<<p.M, 256, 0, st>>>(ra);
     if (kv_only) break;
     AttnArgs aa{c->qf, c->kf, c->vf, c->valid, c->attn, c->po, c->pml, p.B, p.P, p.s_pad, p.n_mt, p.items, p.nsplit};
     prefix_attn_kernel<<<p.B * p.items * p.nsplit, 512, 0, st>>>(aa);
     if (p.nsplit > 1) attn_merge_kernel<<<p.M, 256, 0, st>>>(c->po, c->pml, c->attn, p.B, p.P, p.n_mt, p.nsplit);
-    if (c->o_split) {
-      if ((rc = gemm(c, c->g_osk, w + kPOffO, c->attn, c->dpart, st)) != PI05_OK) return rc;
-      rmsnorm_kernel<<<p.M, 256, 0, st>>>(l == 0 ? emb : c->h, nullptr, ln + kPW, c->h, c->n, eps, c->dpart, kDownSplits, (size_t)p.M * kPW);
-    } else {
-      if ((rc = gemm(c, c->g_o, w + kPOffO, c->attn, c->y, st)) != PI05_OK) return rc;
-      rmsnorm_kernel<<<p.M, 256, 0, st>>>(l == 0 ? emb : c->h, c->y, ln + kPW, c->h, c->n, eps);
-    }
-    if ((rc = gemm(c, c->g_gu, w + kPOffGu, c->n, c->gu, st)) != PI05_OK) return rc;
-    const size_t chunks = (size_t)p.M * (kPI / 8);
-    geglu_kernel<<<(unsigned)((chunks + 255) / 256 < 4096 ? (chunks + 255) / 256 : 4096), 256, 0, st>>>(c->gu, c->act, chunks);
-    if (c->down_split) {
-      if ((rc = gemm(c, c->g_dsk, w + kPOffD, c->act, c->dpart, st)) != PI05_OK) return rc;
-      if (l + 1 < p.L)
-        rmsnorm_kernel<<<p.M, 256, 0, st>>>(c->h, nullptr, c->ln + (size_t)(l + 1) * 2 * kPW, c->h, c->n, eps, c->dpart, kDownSplits,
-                                            (size_t)p.M * kPW);
-    } else {
-      if ((rc = gemm(c, c->g_d, w + kPOffD, c->act, c->y, st)) != PI05_OK) return rc;
-      if (l + 1 < p.L) rmsnorm_kernel<<<p.M, 256, 0, st>>>(c->h, c->y, c->ln + (size_t)(l + 1) * 2 * kPW, c->h, c->n, eps);
-    }
+    if ((rc = residual(c->lib_o, c->g_o, c->m_o, w + kPOffO, c->attn, kPHD, l == 0 ? emb : c->h, ln + kPW)) != PI05_OK) return rc;
+    if ((rc = mm(c, c->m_gu, kMmGeglu, w + kPOffGu, c->n, c->act, kPGuN, kPW, kPI, st)) != PI05_OK) return rc;
+    if ((rc = residual(c->lib_d, c->g_d, c->m_d, w + kPOffD, c->act, kPI, c->h, l + 1 < p.L ? ln + 2 * kPW : nullptr)) != PI05_OK) return rc;
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(c, "prefill launch", e);
+  return PI05_OK;
+}
+
+int pi05_debug_product(int cfg, int epi, const void* a, const void* w, void* c, const float* bias, int M, int N, int K, int lda, int ldw,
+                       int ldc, int split, void* stream) {
+  const MmArgs args{static_cast<const u16*>(a), static_cast<const u16*>(w), c, bias, M, N, K, lda, ldw, ldc, split};
+  if (!a || !w || !c || epi < kMmBf16 || epi > kMmGeglu || !mm_fits(cfg, epi, args)) return fail(nullptr, PI05_E_INVALID, "the tile does not take this product");
+  if (!mm_launch(cfg, epi, args, static_cast<hipStream_t>(stream))) return fail(nullptr, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
 

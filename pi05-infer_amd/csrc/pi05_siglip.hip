@@ -2,13 +2,15 @@
 // gemma_pytorch.py:106-107; the tower itself is transformers' SiglipVisionModel).  Per image:
 //   patches (fp32 im2col) . Wpatch^T          hipBLASLt fp32 GEMM
 //   h = bf16(conv + bpatch + pos)              embed_kernel
-//   27 x [ n = LN1(h); q|k|v = n.W^T + b      hipBLASLt (bias epilogue)
+//   27 x [ n = LN1(h); q|k|v = n.W^T + b      product (bias epilogue)
 //          attention, 16 heads of 72          vision_attn_kernel (MFMA, K/V staged in LDS)
-//          h = bf16(h + o.Wo^T + bo); n = LN2 hipBLASLt (split-K when faster) + layernorm_kernel
-//          a = gelu_tanh(n.W1^T + b1)          hipBLASLt + gelu_kernel
-//          h = bf16(h + a.W2^T + b2) ]         hipBLASLt (split-K when faster) + layernorm_kernel
+//          h = bf16(h + o.Wo^T + bo); n = LN2 product (split-K when faster) + layernorm_kernel
+//          a = gelu_tanh(n.W1^T + b1)          product (bias and GELU epilogue)
+//          h = bf16(h + a.W2^T + b2) ]         product (split-K when faster) + layernorm_kernel
 //                                              (the next LN1 / post_layernorm)
-//   out = (n.Wproj^T + bproj) * out_scale     hipBLASLt (+ scale_kernel)
+//   out = (n.Wproj^T + bproj) * out_scale     product (+ scale_kernel)
+// The bf16 products run on pi05_mm.h; from kVLibRows rows on, q|k|v, out_proj, fc2 and the projector on
+// hipBLASLt where it measured faster when the context was created.
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 
@@ -19,6 +21,7 @@
 
 #include "pi05_blocks.h"
 #include "pi05_gemm.h"
+#include "pi05_mm.h"
 #include "pi05_siglip.h"
 
 namespace pi05 {
@@ -43,7 +46,9 @@ constexpr size_t kVPOffBqkv = 0, kVPOffBo = kVQkvN, kVPOffB1 = kVPOffBo + kVW, k
                  kVPOffLn1w = kVPOffB2 + kVW, kVPOffLn1b = kVPOffLn1w + kVW, kVPOffLn2w = kVPOffLn1b + kVW,
                  kVPOffLn2b = kVPOffLn2w + kVW, kVLayerParams = kVPOffLn2b + kVW;
 constexpr size_t kVWorkspace = 32ull << 20;
-constexpr int kVMaxSplits = 8;  // split-K candidates: 4 and 8 K slices (out_proj, fc2); 2 and 3 (fc1)
+constexpr int kVMaxSplits = 8;  // K splits of out_proj and fc2 at most
+// rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate
+constexpr int kVLibRows = 1024;
 
 thread_local std::string g_vision_err;
 
@@ -269,41 +274,6 @@ __global__ __launch_bounds__(512) void vision_attn_kernel(const u16* qkv, u16* o
     }
 }
 
-// bf16(gelu_tanh(x)) in place (transformers' gelu_pytorch_tanh on the bf16 fc1 output)
-// (8 elements per thread over the padded rows; chunks = elements / 8)
-__global__ __launch_bounds__(256) void gelu_kernel(u16* x, size_t chunks) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < chunks; i += (size_t)gridDim.x * 256) {
-    u16x8 v = *reinterpret_cast<const u16x8*>(x + i * 8);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = f2bf(gelu_tanh(bf2f(v[e])));
-    *reinterpret_cast<u16x8*>(x + i * 8) = v;
-  }
-}
-
-// act = bf16(gelu_tanh(bf16(sum of nsplit fp32 fc1 partials + b1))): fc1 run as a split-K GEMM,
-// reduced here with its bias and the one rounding a GEMM epilogue would apply; the pad columns of
-// the 4352-wide rows are written as zeros.
-__global__ __launch_bounds__(256) void gelu_split_kernel(const float* part, int nsplit, size_t split_stride, const float* bias, u16* act,
-                                                        size_t chunks) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < chunks; i += (size_t)gridDim.x * 256) {
-    const int col = (int)((i * 8) % kVIp);
-    u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (col < kVI) {
-      float a[8];
-      const float4 p0 = *reinterpret_cast<const float4*>(part + i * 8), p1 = *reinterpret_cast<const float4*>(part + i * 8 + 4);
-      a[0] = p0.x, a[1] = p0.y, a[2] = p0.z, a[3] = p0.w, a[4] = p1.x, a[5] = p1.y, a[6] = p1.z, a[7] = p1.w;
-      for (int sp = 1; sp < nsplit; ++sp) {
-        const float* q = part + (size_t)sp * split_stride + i * 8;
-        const float4 q0 = *reinterpret_cast<const float4*>(q), q1 = *reinterpret_cast<const float4*>(q + 4);
-        a[0] += q0.x, a[1] += q0.y, a[2] += q0.z, a[3] += q0.w, a[4] += q1.x, a[5] += q1.y, a[6] += q1.z, a[7] += q1.w;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = f2bf(gelu_tanh(round_bf(fadd(a[e], bias[col + e]))));
-    }
-    *reinterpret_cast<u16x8*>(act + i * 8) = v;
-  }
-}
-
 __global__ __launch_bounds__(256) void scale_kernel(u16* x, size_t total, float s) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) x[i] = f2bf(bf2f(x[i]) * s);
 }
@@ -334,7 +304,7 @@ VisionPlan vplan_of(const pi05_vision_dims& d) {
   p.head = vrup(((size_t)kVW * kVPD + kVW + (size_t)kVS * kVW + 2 * kVW + kVProj) * 4 + (size_t)kVProj * kVW * 2);
   p.h = vrup(M * kVW * 2);
   p.qkv = vrup(M * kVQkvN * 2);
-  p.part = vrup(std::max((size_t)kVMaxSplits * M * kVW, (size_t)3 * M * kVIp) * 4);
+  p.part = vrup((size_t)kVMaxSplits * M * kVW * 4);
   p.act = vrup(M * kVIp * 2);
   p.patches = vrup(M * kVPD * 4);
   p.conv = vrup(M * kVW * 4);
@@ -363,13 +333,6 @@ bool check_vision_dims(const pi05_vision_dims* d, std::string* m) {
   return true;
 }
 
-GemmOpts split_opts(int nsplit, int ld_k) {
-  GemmOpts o;
-  o.batch = nsplit;
-  o.ld_k = ld_k;
-  return o;
-}
-
 unsigned grid_for(size_t total) {
   const size_t g = (total + 255) / 256;
   return (unsigned)(g < 8192 ? g : 8192);
@@ -394,11 +357,10 @@ struct pi05_vision_ctx {
         *part = nullptr, *patches = nullptr, *conv = nullptr;
   void* ws = nullptr;
   hipblasLtHandle_t lt = nullptr;
-  GemmPlan g_patch, g_qkv, g_o, g_fc1, g_fc2, g_proj;
-  // out_proj / fc2 as fp32 split-K GEMMs (4 or 8 K slices) reduced in the LayerNorm, when faster
-  GemmPlan g_osk[2], g_fc2sk[2];
-  GemmPlan g_fc1sk[2];  // fc1 as 2 or 3 fp32 split-K GEMMs reduced (+ bias, GELU) in gelu_split_kernel
-  int o_split = 0, fc2_split = 0, fc1_split = 0;  // chosen slice count (0: the single bf16 GEMM with its bias)
+  // the bf16 products: on pi05_mm.h, or (from kVLibRows rows, where it measured faster) on hipBLASLt
+  GemmPlan g_patch, g_qkv, g_o, g_fc2, g_proj;
+  MmPlan m_qkv, m_o, m_fc1, m_fc2, m_proj;
+  bool lib_qkv = false, lib_o = false, lib_fc2 = false, lib_proj = false;
 };
 
 namespace {
@@ -412,6 +374,12 @@ int vfail(pi05_vision_ctx* c, int code, const std::string& m) {
 int vgemm(pi05_vision_ctx* c, const GemmPlan& p, const void* W, const void* A, void* C, const float* bias, hipStream_t st) {
   const hipblasStatus_t s = run_plan(c->lt, p, p.algo, p.ws, W, A, C, bias, c->ws, st);
   if (!lt_ok(s)) return vfail(c, PI05_E_HIP, "hipblasLtMatmul failed (status " + std::to_string((int)s) + ")");
+  return PI05_OK;
+}
+
+int vmm(pi05_vision_ctx* c, const MmPlan& p, int epi, MmArgs a, hipStream_t st) {
+  a.split = p.split;
+  if (!mm_launch(p.cfg, epi, a, st)) return vfail(c, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
 
@@ -500,51 +468,46 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   f32.c = HIP_R_32F;
   GemmOpts bias;
   bias.bias = true;
-  GemmOpts fc1o = bias;
-  fc1o.ld_c = kVIp;
   GemmOpts fc2o = bias;
   fc2o.ld_k = kVIp;
-  constexpr int splits[2] = {4, 8};
-  static_assert(splits[0] <= kVMaxSplits && splits[1] <= kVMaxSplits, "layernorm_kernel reduces at most kVMaxSplits slices");
+  const bool lib = M > kVLibRows;
   bool ok = lt_ok(hipblasLtCreate(&c->lt)) && make_plan(c->lt, M, kVW, kVPD, kVWorkspace, &c->g_patch, &perr, f32) &&
-            make_plan(c->lt, M, kVQkvN, kVW, kVWorkspace, &c->g_qkv, &perr, bias) && make_plan(c->lt, M, kVW, kVW, kVWorkspace, &c->g_o, &perr, bias) &&
-            make_plan(c->lt, M, kVI, kVW, kVWorkspace, &c->g_fc1, &perr, fc1o) && make_plan(c->lt, M, kVW, kVIp, kVWorkspace, &c->g_fc2, &perr, fc2o) &&
-            make_plan(c->lt, M, kVProj, kVW, kVWorkspace, &c->g_proj, &perr, bias);
-  const int fc1_splits[2] = {2, 3};
-  for (int i = 0; i < 2 && ok; ++i) {
-    GemmOpts f1 = split_opts(fc1_splits[i], kVW);
-    f1.ld_c = kVIp;
-    ok = make_plan(c->lt, M, kVW, kVW / splits[i], kVWorkspace, &c->g_osk[i], &perr, split_opts(splits[i], kVW)) &&
-         make_plan(c->lt, M, kVW, kVIp / splits[i], kVWorkspace, &c->g_fc2sk[i], &perr, split_opts(splits[i], kVIp)) &&
-         make_plan(c->lt, M, kVI, kVW / fc1_splits[i], kVWorkspace, &c->g_fc1sk[i], &perr, f1);
-  }
+            (!lib || (make_plan(c->lt, M, kVQkvN, kVW, kVWorkspace, &c->g_qkv, &perr, bias) && make_plan(c->lt, M, kVW, kVW, kVWorkspace, &c->g_o, &perr, bias) &&
+                      make_plan(c->lt, M, kVW, kVIp, kVWorkspace, &c->g_fc2, &perr, fc2o) && make_plan(c->lt, M, kVProj, kVW, kVWorkspace, &c->g_proj, &perr, bias)));
   if (ok) {
     const float* bz = c->par;  // any fp32 vector long enough (zeros) stands in for the biases while timing
     // (weights rotate over the layers' blocks while timing, as the layer loop streams them)
     const size_t ls = kVLayerElems * 2;
     const int nl = p.L;
+    // what a reader of fp32 partials pays per split: 4 bytes per output element at ~4 TB/s, less the
+    // bf16 output it would read and the product write otherwise
+    const float part_ms = (float)(4.0 * M * kVW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kVW / 4e12 * 1e3);
     ok = tune_plan(c->lt, &c->g_patch, c->patch_w, c->patches, c->conv, c->ws, nullptr) &&
-         tune_plan(c->lt, &c->g_qkv, c->w, c->n, c->qkv, c->ws, nullptr, bz, ls, nl) &&
-         tune_plan(c->lt, &c->g_o, c->w, c->attn, c->y, c->ws, nullptr, bz, ls, nl) &&
-         tune_plan(c->lt, &c->g_fc1, c->w, c->n, c->act, c->ws, nullptr, bz, ls, nl) &&
-         tune_plan(c->lt, &c->g_fc2, c->w, c->act, c->y, c->ws, nullptr, bz, ls, nl) &&
-         tune_plan(c->lt, &c->g_proj, c->proj_w, c->n, c->act, c->ws, nullptr, bz);
-    for (int i = 0; i < 2 && ok; ++i)
-      ok = tune_plan(c->lt, &c->g_osk[i], c->w, c->attn, c->part, c->ws, nullptr, nullptr, ls, nl) &&
-           tune_plan(c->lt, &c->g_fc2sk[i], c->w, c->act, c->part, c->ws, nullptr, nullptr, ls, nl) &&
-           tune_plan(c->lt, &c->g_fc1sk[i], c->w, c->n, c->part, c->ws, nullptr, nullptr, ls, nl);
-    if (!ok && perr.empty()) perr = "GEMM algorithm tuning failed";
-    // split-K when the split GEMM plus the partials' extra traffic through the LayerNorm
-    // ((4 nsplit - 2) bytes per output element at ~4 TB/s) beats the single bf16 GEMM
-    auto extra_ms = [&](int ns) { return (float)((double)(4 * ns - 2) * M * kVW / 4e12 * 1e3); };
-    float best_o = c->g_o.ms, best_2 = c->g_fc2.ms, best_1 = c->g_fc1.ms;
-    for (int i = 0; i < 2 && ok; ++i) {
-      // fc1: the partials replace the bf16 output that the GELU reads anyway
-      const float x1 = (float)((double)(4 * fc1_splits[i] - 2) * M * kVIp / 4e12 * 1e3);
-      if (c->g_fc1sk[i].ms + x1 < best_1) best_1 = c->g_fc1sk[i].ms + x1, c->fc1_split = fc1_splits[i];
-      if (c->g_osk[i].ms + extra_ms(splits[i]) < best_o) best_o = c->g_osk[i].ms + extra_ms(splits[i]), c->o_split = splits[i];
-      if (c->g_fc2sk[i].ms + extra_ms(splits[i]) < best_2) best_2 = c->g_fc2sk[i].ms + extra_ms(splits[i]), c->fc2_split = splits[i];
+         mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+         mm_tune({c->n, c->w, c->act, bz, M, kVI, kVW, kVW, kVW, kVIp, 1}, kMmGelu, 1, 1, 0.f, ls, nl, nullptr, &c->m_fc1) &&
+         mm_tune({c->n, c->proj_w, c->act, bz, M, kVProj, kVW, kVW, kVW, kVProj, 1}, kMmBf16, 1, 1, 0.f, 0, 1, nullptr, &c->m_proj);
+    // out_proj and fc2: one product with its bias, or fp32 K splits that the LayerNorm adds
+    auto tune_n = [&](const u16* A, int K, MmPlan* out) {
+      MmPlan one, sp;
+      if (!mm_tune({A, c->w, c->y, bz, M, kVW, K, K, K, kVW, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &one) ||
+          !mm_tune({A, c->w, c->part, nullptr, M, kVW, K, K, K, kVW, 1}, kMmF32, 2, kVMaxSplits, part_ms, ls, nl, nullptr, &sp))
+        return false;
+      *out = sp.ms + part_ms * (float)sp.split - bf_ms < one.ms ? sp : one;
+      return true;
+    };
+    ok = ok && tune_n(c->attn, kVW, &c->m_o) && tune_n(c->act, kVIp, &c->m_fc2);
+    if (ok && lib) {
+      ok = tune_plan(c->lt, &c->g_qkv, c->w, c->n, c->qkv, c->ws, nullptr, bz, ls, nl) &&
+           tune_plan(c->lt, &c->g_o, c->w, c->attn, c->y, c->ws, nullptr, bz, ls, nl) &&
+           tune_plan(c->lt, &c->g_fc2, c->w, c->act, c->y, c->ws, nullptr, bz, ls, nl) &&
+           tune_plan(c->lt, &c->g_proj, c->proj_w, c->n, c->act, c->ws, nullptr, bz);
+      auto cost = [&](const MmPlan& m) { return m.split > 1 ? m.ms + part_ms * (float)m.split - bf_ms : m.ms; };
+      c->lib_qkv = c->g_qkv.ms < c->m_qkv.ms;
+      c->lib_o = c->g_o.ms < cost(c->m_o);
+      c->lib_fc2 = c->g_fc2.ms < cost(c->m_fc2);
+      c->lib_proj = c->g_proj.ms < c->m_proj.ms;
     }
+    if (!ok && perr.empty()) perr = "GEMM tuning failed";
   }
   if (!ok) {
     if (perr.empty()) perr = "hipblasLtCreate failed";
@@ -557,8 +520,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
 
 int pi05_vision_destroy(pi05_vision_ctx* c) {
   if (!c) return PI05_OK;
-  for (GemmPlan* g : {&c->g_patch, &c->g_qkv, &c->g_o, &c->g_fc1, &c->g_fc2, &c->g_proj, &c->g_osk[0], &c->g_osk[1], &c->g_fc2sk[0],
-                      &c->g_fc2sk[1], &c->g_fc1sk[0], &c->g_fc1sk[1]})
+  for (GemmPlan* g : {&c->g_patch, &c->g_qkv, &c->g_o, &c->g_fc2, &c->g_proj})
     free_plan(g);
   if (c->lt) hipblasLtDestroy(c->lt);
   if (c->base) hipFree(c->base);
@@ -662,40 +624,36 @@ int pi05_vision_forward(pi05_vision_ctx* c, const float* pixels, void* out, void
   const unsigned ln_grid = (unsigned)((M + 3) / 4);
   const size_t pstride = M * kVW;
   layernorm_kernel<<<ln_grid, 256, 0, st>>>(c->h, nullptr, nullptr, 0, 0, nullptr, pr0 + kVPOffLn1w, pr0 + kVPOffLn1b, nullptr, c->n, eps, (int)M);
+  const int iM = (int)M;
+  // h += A . W^T + bias, n = LayerNorm(h)
+  auto residual = [&](bool lib, const GemmPlan& g, const MmPlan& m, const u16* A, int K, const u16* W, const float* bias, const float* nw,
+                      const float* nb) {
+    const bool parts = !lib && m.split > 1;
+    const int e = lib ? vgemm(c, g, W, A, c->y, bias, st)
+                      : parts ? vmm(c, m, kMmF32, {A, W, c->part, nullptr, iM, kVW, K, K, K, kVW, 1}, st)
+                              : vmm(c, m, kMmBf16, {A, W, c->y, bias, iM, kVW, K, K, K, kVW, 1}, st);
+    if (e != PI05_OK) return e;
+    layernorm_kernel<<<ln_grid, 256, 0, st>>>(c->h, parts ? nullptr : c->y, parts ? c->part : nullptr, parts ? m.split : 0, pstride,
+                                              parts ? bias : nullptr, nw, nb, c->h, c->n, eps, iM);
+    return (int)PI05_OK;
+  };
   for (int l = 0; l < p.L; ++l) {
     const u16* w = c->w + (size_t)l * kVLayerElems;
     const float* pr = c->par + (size_t)l * kVLayerParams;
-    if ((rc = vgemm(c, c->g_qkv, w + kVOffQkv, c->n, c->qkv, pr + kVPOffBqkv, st)) != PI05_OK) return rc;
+    rc = c->lib_qkv ? vgemm(c, c->g_qkv, w + kVOffQkv, c->n, c->qkv, pr + kVPOffBqkv, st)
+                    : vmm(c, c->m_qkv, kMmBf16, {c->n, w + kVOffQkv, c->qkv, pr + kVPOffBqkv, iM, kVQkvN, kVW, kVW, kVW, kVQkvN, 1}, st);
+    if (rc != PI05_OK) return rc;
     vision_attn_kernel<<<(unsigned)(p.N * kVH * 2), 512, 0, st>>>(c->qkv, c->attn);
-    if (c->o_split) {
-      if ((rc = vgemm(c, c->g_osk[c->o_split == 8], w + kVOffO, c->attn, c->part, nullptr, st)) != PI05_OK) return rc;
-      layernorm_kernel<<<ln_grid, 256, 0, st>>>(c->h, nullptr, c->part, c->o_split, pstride, pr + kVPOffBo, pr + kVPOffLn2w,
-                                                pr + kVPOffLn2b, c->h, c->n, eps, (int)M);
-    } else {
-      if ((rc = vgemm(c, c->g_o, w + kVOffO, c->attn, c->y, pr + kVPOffBo, st)) != PI05_OK) return rc;
-      layernorm_kernel<<<ln_grid, 256, 0, st>>>(c->h, c->y, nullptr, 0, 0, nullptr, pr + kVPOffLn2w, pr + kVPOffLn2b, c->h, c->n, eps,
-                                                (int)M);
-    }
-    if (c->fc1_split) {
-      if ((rc = vgemm(c, c->g_fc1sk[c->fc1_split == 3], w + kVOff1, c->n, c->part, nullptr, st)) != PI05_OK) return rc;
-      gelu_split_kernel<<<grid_for(M * kVIp / 8), 256, 0, st>>>(c->part, c->fc1_split, M * kVIp, pr + kVPOffB1, c->act, M * kVIp / 8);
-    } else {
-      if ((rc = vgemm(c, c->g_fc1, w + kVOff1, c->n, c->act, pr + kVPOffB1, st)) != PI05_OK) return rc;
-      gelu_kernel<<<grid_for(M * kVIp / 8), 256, 0, st>>>(c->act, M * kVIp / 8);
-    }
+    if ((rc = residual(c->lib_o, c->g_o, c->m_o, c->attn, kVW, w + kVOffO, pr + kVPOffBo, pr + kVPOffLn2w, pr + kVPOffLn2b)) != PI05_OK) return rc;
+    if ((rc = vmm(c, c->m_fc1, kMmGelu, {c->n, w + kVOff1, c->act, pr + kVPOffB1, iM, kVI, kVW, kVW, kVW, kVIp, 1}, st)) != PI05_OK) return rc;
     const bool last = l + 1 == p.L;
     const float* nw = last ? c->post_w : c->par + (size_t)(l + 1) * kVLayerParams + kVPOffLn1w;
     const float* nb = last ? c->post_b : c->par + (size_t)(l + 1) * kVLayerParams + kVPOffLn1b;
-    if (c->fc2_split) {
-      if ((rc = vgemm(c, c->g_fc2sk[c->fc2_split == 8], w + kVOff2, c->act, c->part, nullptr, st)) != PI05_OK) return rc;
-      layernorm_kernel<<<ln_grid, 256, 0, st>>>(c->h, nullptr, c->part, c->fc2_split, pstride, pr + kVPOffB2, nw, nb, c->h, c->n, eps,
-                                                (int)M);
-    } else {
-      if ((rc = vgemm(c, c->g_fc2, w + kVOff2, c->act, c->y, pr + kVPOffB2, st)) != PI05_OK) return rc;
-      layernorm_kernel<<<ln_grid, 256, 0, st>>>(c->h, c->y, nullptr, 0, 0, nullptr, nw, nb, c->h, c->n, eps, (int)M);
-    }
+    if ((rc = residual(c->lib_fc2, c->g_fc2, c->m_fc2, c->act, kVIp, w + kVOff2, pr + kVPOffB2, nw, nb)) != PI05_OK) return rc;
   }
-  if ((rc = vgemm(c, c->g_proj, c->proj_w, c->n, out, c->proj_b, st)) != PI05_OK) return rc;
+  rc = c->lib_proj ? vgemm(c, c->g_proj, c->proj_w, c->n, out, c->proj_b, st)
+                   : vmm(c, c->m_proj, kMmBf16, {c->n, c->proj_w, out, c->proj_b, iM, kVProj, kVW, kVW, kVW, kVProj, 1}, st);
+  if (rc != PI05_OK) return rc;
   if (c->d.out_scale != 1.0f) scale_kernel<<<grid_for(M * kVProj), 256, 0, st>>>(static_cast<u16*>(out), M * kVProj, c->d.out_scale);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return vfail(c, PI05_E_HIP, std::string("vision launch: ") + hipGetErrorString(e));

@@ -68,6 +68,7 @@ PREFIX_EXPORTED_SYMBOLS = (
     "pi05_prefix_embed_tokens",
     "pi05_prefix_status",
     "pi05_prefix_forward",
+    "pi05_debug_product",
 )
 
 # every exported symbol of include/pi05_siglip.h
@@ -226,6 +227,7 @@ def load_prefix_library(path: str = PREFIX_LIB_PATH) -> ctypes.CDLL:
         "pi05_prefix_refresh_weights": (i32, [vp, vp]),
         "pi05_prefix_embed_tokens": (i32, [vp, vp, i64, vp, i64, vp, vp]),
         "pi05_prefix_status": (i32, [vp, vp]),
+        "pi05_debug_product": (i32, [i32, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, vp]),
         "pi05_prefix_forward": (i32, [vp, vp, vp, ctypes.POINTER(vp), ctypes.POINTER(vp), i64, i64, vp]),
         "pi05_vision_default_dims": (None, [vdims_p]),
         "pi05_vision_check_dims": (i32, [vdims_p]),
