@@ -199,13 +199,22 @@ struct MmInt {
   static constexpr int v = V;
 };
 
-// Workgroup -> (m-tile, n-tile, split).  Workgroups are dealt round-robin over the 8 XCDs, so XCD x takes
-// one contiguous run of tiles; the run walks bands of up to kMmBand m-tiles, m fastest, so the 32 tiles an
-// XCD works on at a time share few rows of A and of W in its L2.
+// Tiles are numbered in bands of up to kMmBand m-tiles, m fastest, one K split after the other, and XCD x takes
+// one contiguous run of them (workgroups are dealt round-robin over the 8 XCDs): the 32 tiles an XCD works on
+// at a time share few rows of A and of W in its L2.  Workgroup w of the g
+// on XCD x takes the run's tiles w, w + g, ...: with one workgroup per tile exactly one, as a run of n tiles
+// has n workgroups then.
 constexpr int kMmBand = 6;
-__device__ __forceinline__ void mm_tile(const MmArgs& a, int bm, int bn, int& mt, int& nt, int& sp) {
-  const int g = gridDim.x, x = blockIdx.x & 7, q = g >> 3, r = g & 7;
-  int id = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
+__device__ __forceinline__ int mm_tiles(const MmArgs& a, int bm, int bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.split; }
+__device__ __forceinline__ int mm_last(int tiles) {
+  const int x = blockIdx.x & 7, r = tiles & 7;
+  return (x + 1) * (tiles >> 3) + (x + 1 < r ? x + 1 : r);
+}
+__device__ __forceinline__ int mm_first(int tiles) {
+  const int x = blockIdx.x & 7, r = tiles & 7;
+  return x * (tiles >> 3) + (x < r ? x : r) + (blockIdx.x >> 3);
+}
+__device__ __forceinline__ void mm_tile(const MmArgs& a, int bm, int bn, int id, int& mt, int& nt, int& sp) {
   const int tm = (a.M + bm - 1) / bm, tn = (a.N + bn - 1) / bn;
   sp = id / (tm * tn);
   id -= sp * tm * tn;
@@ -213,6 +222,15 @@ __device__ __forceinline__ void mm_tile(const MmArgs& a, int bm, int bn, int& mt
   id -= band * kMmBand * tn;
   mt = band * kMmBand + id % h;
   nt = id / h;
+}
+
+// gelu_tanh(x) = x (1 + tanh(u)) / 2 = x / (1 + exp(-2 u)), u = sqrt(2 / pi) (x + 0.044715 x^3): one hardware exp2 and
+// reciprocal and five other operations.  The epilogues evaluate it 64 times a lane with the matrix cores
+// idle (gelu_tanh's fourteen operations: 6 us of a 256 x 256 tile's 55).
+__device__ __forceinline__ float mm_gelu(float x) {
+  const float k = -2.0f * 0.7978845608028654f * 1.4426950408889634f;  // exp(-2 u) = exp2(k (x + 0.044715 x^3))
+  const float e = __builtin_amdgcn_exp2f(x * __builtin_fmaf(x * x, k * 0.044715f, k));
+  return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
 // The epilogue of four columns col .. col + 3 of one row.
@@ -227,14 +245,14 @@ __device__ __forceinline__ void mm_store(const MmArgs& a, int sp, int row, int c
     }
     u16x4 o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = EPI == kMmGelu ? f2bf(gelu_tanh(round_bf(v[i]))) : f2bf(v[i]);
+    for (int i = 0; i < 4; ++i) o[i] = EPI == kMmGelu ? f2bf(mm_gelu(round_bf(v[i]))) : f2bf(v[i]);
     *reinterpret_cast<u16x4*>(static_cast<u16*>(a.C) + (size_t)row * a.ldc + col) = o;
   }
 }
 __device__ __forceinline__ void mm_store_geglu(const MmArgs& a, int row, int col, f32x4 g, f32x4 u) {
   u16x4 o;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = f2bf(fmul(gelu_tanh(round_bf(g[i])), round_bf(u[i])));
+  for (int i = 0; i < 4; ++i) o[i] = f2bf(fmul(mm_gelu(round_bf(g[i])), round_bf(u[i])));
   *reinterpret_cast<u16x4*>(static_cast<u16*>(a.C) + (size_t)row * a.ldc + col) = o;
 }
 
@@ -261,17 +279,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __shared__ __align__(1024) uint8_t lds[AS * kA + WS * kW];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wave >> 2, wn = wave & 3;
-  int m_t, n_t, sp;
-  mm_tile(a, BM, BN, m_t, n_t, sp);
-  const int m0 = m_t * BM, n0 = n_t * BN;
-  const int t0 = sp * (a.K / 64) / a.split, T = (sp + 1) * (a.K / 64) / a.split - t0;
-  const mm_rsrc ra = mm_make_rsrc(a.A + (size_t)m0 * a.lda + t0 * 64), rw = mm_make_rsrc(a.W + (size_t)n0 * a.ldw + t0 * 64);
-  int va[PA], vw[PW];
-#pragma unroll
-  for (int i = 0; i < PA; ++i) va[i] = mm_src(grp * (BM / 2) + (i * 4 + wn) * 8 + (lane >> 3), a.M - 1 - m0, a.lda, lane);
-#pragma unroll
-  for (int i = 0; i < PW; ++i) vw[i] = mm_src((i * 8 + wave) * 8 + (lane >> 3), a.N - 1 - n0, a.ldw, lane);
   mm_lds* ldsb = (mm_lds*)lds;
+  const uint32_t base = (uint32_t)(uintptr_t)ldsb;
+  const int fr = lane & 15, fg = lane >> 4;
+  const uint32_t ao = base + (grp * (BM / 2) + fr) * 128, wo = base + AS * kA + (wn * (BN / 4) + fr) * 128;
+  const uint32_t x0 = (fg ^ (fr & 7)) * 16, x1 = ((4 + fg) ^ (fr & 7)) * 16;
+  constexpr int kMax = AS > WS ? AS : WS;
+  // copies that may still be in flight when a slot ends (a wave's loads complete in order): after the
+  // group's own A(t + 1), after W(t + 1), after both
+  constexpr int wa = PW + (AS - 2) * PT, wb = (WS - 2) * PT, wab = wa < wb ? wa : wb;
+  // the tile being multiplied; its operands' copies
+  int m0, n0, sp, T;
+  mm_rsrc ra, rw;
+  int va[PA], vw[PW];
   auto cp_a = [&](int kt, int st) {
 #pragma unroll
     for (int i = 0; i < PA; ++i)
@@ -282,70 +302,90 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < PW; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, ldsb + AS * (kA / 2) + st * (kW / 2) + (i * 8 + wave) * 512, 16, vw[i], kt * 128, 0, 0);
   };
-  const uint32_t base = (uint32_t)(uintptr_t)ldsb;
-  const int fr = lane & 15, fg = lane >> 4;
-  const uint32_t ao = base + (grp * (BM / 2) + fr) * 128, wo = base + AS * kA + (wn * (BN / 4) + fr) * 128;
-  const uint32_t x0 = (fg ^ (fr & 7)) * 16, x1 = ((4 + fg) ^ (fr & 7)) * 16;
-  f32x4 acc[FN][FM];
+  // sets out on tile id: its first copies, M(1 - kMax) .. M(-1)
+  auto begin = [&](int id) {
+    int m_t, n_t;
+    mm_tile(a, BM, BN, id, m_t, n_t, sp);
+    m0 = m_t * BM, n0 = n_t * BN;
+    const int t0 = sp * (a.K / 64) / a.split;
+    T = (sp + 1) * (a.K / 64) / a.split - t0;
+    ra = mm_make_rsrc(a.A + (size_t)m0 * a.lda + t0 * 64), rw = mm_make_rsrc(a.W + (size_t)n0 * a.ldw + t0 * 64);
 #pragma unroll
-  for (int n = 0; n < FN; ++n)
+    for (int i = 0; i < PA; ++i) va[i] = mm_src(grp * (BM / 2) + (i * 4 + wn) * 8 + (lane >> 3), a.M - 1 - m0, a.lda, lane);
 #pragma unroll
-    for (int m = 0; m < FM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  MmFrags<FM, FN> f;
-  constexpr int kMax = AS > WS ? AS : WS;
-  // copies that may still be in flight when a slot ends (a wave's loads complete in order): after the
-  // group's own A(t + 1), after W(t + 1), after both
-  constexpr int wa = PW + (AS - 2) * PT, wb = (WS - 2) * PT, wab = wa < wb ? wa : wb;
+    for (int i = 0; i < PW; ++i) vw[i] = mm_src((i * 8 + wave) * 8 + (lane >> 3), a.N - 1 - n0, a.ldw, lane);
 #pragma unroll
-  for (int s = 1 - kMax; s < 0; ++s) {
-    if (s + AS - 1 >= 0 && s + AS - 1 < T) cp_a(s + AS - 1, s + AS - 1);
-    if (s + WS - 1 >= 0 && s + WS - 1 < T) cp_w(s + WS - 1, s + WS - 1);
-  }
-  int as = 0, ws = 0, al = AS - 1, wl = WS - 1;  // ring slots of the tile being read, of the next copies
-  int t = 0;
-  if (T >= kMax) mm_wait_vm<wab>();
-  else mm_wait_vm<0>();
-  mm_barrier();
-  // kIn: every copy of the step exists, w0 / w1 / w2 may stay in flight (group 0's C, group 1's M and C)
-  auto step = [&](auto kin, auto w0, auto w1, auto w2) {
-    if (decltype(kin)::v || t + AS - 1 < T) cp_a(t + AS - 1, al);
-    if (decltype(kin)::v || t + WS - 1 < T) cp_w(t + WS - 1, wl);
-    const uint32_t sa = as * kA, sw = ws * kW;
-    f.load(ao + x0 + sa, ao + x1 + sa, wo + x0 + sw, wo + x1 + sw);
-    if (grp) mm_wait_vm<decltype(w1)::v>();
-    mm_barrier();
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int n = 0; n < FN; ++n)
-#pragma unroll
-        for (int m = 0; m < FM; ++m) acc[n][m] = mfma16x16x32(f.w[ks][n], f.a[ks][m], acc[n][m]);
-    __builtin_amdgcn_s_setprio(0);
-    if (grp) mm_wait_vm<decltype(w2)::v>();
-    else mm_wait_vm<decltype(w0)::v>();
-    mm_barrier();
-    as = as + 1 == AS ? 0 : as + 1, al = al + 1 == AS ? 0 : al + 1;
-    ws = ws + 1 == WS ? 0 : ws + 1, wl = wl + 1 == WS ? 0 : wl + 1;
-  };
-  if (grp) mm_barrier();
-  for (; t < T - kMax + 1; ++t) step(MmInt<1>{}, MmInt<wab>{}, MmInt<wb>{}, MmInt<wa>{});
-  for (; t < T; ++t) step(MmInt<0>{}, MmInt<0>{}, MmInt<0>{}, MmInt<0>{});
-  if (!grp) mm_barrier();
-  // lane l: columns 16 n + 4 (l / 16) .. + 3 of row l % 16
-#pragma unroll
-  for (int m = 0; m < FM; ++m) {
-    const int row = m0 + grp * (BM / 2) + m * 16 + fr, col = n0 + wn * (BN / 4);
-    if (row >= a.M) continue;
-    if constexpr (EPI == kMmGeglu) {
-#pragma unroll
-      for (int n = 0; n < FN; n += 2)
-        if (col + n * 16 < a.N) mm_store_geglu(a, row, (col + n * 16) / 2 + fg * 4, acc[n][m], acc[n + 1][m]);
-    } else {
-#pragma unroll
-      for (int n = 0; n < FN; ++n)
-        if (col + n * 16 < a.N) mm_store<EPI>(a, sp, row, col + n * 16 + fg * 4, acc[n][m]);
+    for (int s = 1 - kMax; s < 0; ++s) {
+      if (s + AS - 1 >= 0 && s + AS - 1 < T) cp_a(s + AS - 1, s + AS - 1);
+      if (s + WS - 1 >= 0 && s + WS - 1 < T) cp_w(s + WS - 1, s + WS - 1);
     }
+  };
+  const int tiles = mm_tiles(a, BM, BN);
+  int id = mm_first(tiles);
+  const int stride = ((int)gridDim.x + 7 - (int)(blockIdx.x & 7)) >> 3, last = mm_last(tiles);  // stride: this XCD's workgroups, at least one
+  begin(id);
+  mm_wait_vm<wab>();
+  for (;;) {
+    f32x4 acc[FN][FM];
+#pragma unroll
+    for (int n = 0; n < FN; ++n)
+#pragma unroll
+      for (int m = 0; m < FM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    MmFrags<FM, FN> f;
+    int as = 0, ws = 0, al = AS - 1, wl = WS - 1;  // ring slots of the tile being read, of the next copies
+    int t = 0;
+    if (T < kMax) mm_wait_vm<0>();
+    mm_barrier();
+    // kin: every copy of the step exists; w0 / w1 / w2 may stay in flight (group 0's C, group 1's M and C)
+    auto step = [&](auto kin, auto w0, auto w1, auto w2) {
+      if (decltype(kin)::v || t + AS - 1 < T) cp_a(t + AS - 1, al);
+      if (decltype(kin)::v || t + WS - 1 < T) cp_w(t + WS - 1, wl);
+      const uint32_t sa = as * kA, sw = ws * kW;
+      f.load(ao + x0 + sa, ao + x1 + sa, wo + x0 + sw, wo + x1 + sw);
+      if (grp) mm_wait_vm<decltype(w1)::v>();
+      mm_barrier();
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int n = 0; n < FN; ++n)
+#pragma unroll
+          for (int m = 0; m < FM; ++m) acc[n][m] = mfma16x16x32(f.w[ks][n], f.a[ks][m], acc[n][m]);
+      __builtin_amdgcn_s_setprio(0);
+      if (grp) mm_wait_vm<decltype(w2)::v>();
+      else mm_wait_vm<decltype(w0)::v>();
+      mm_barrier();
+      as = as + 1 == AS ? 0 : as + 1, al = al + 1 == AS ? 0 : al + 1;
+      ws = ws + 1 == WS ? 0 : ws + 1, wl = wl + 1 == WS ? 0 : wl + 1;
+    };
+    if (grp) mm_barrier();
+    for (; t < T - kMax + 1; ++t) step(MmInt<1>{}, MmInt<wab>{}, MmInt<wb>{}, MmInt<wa>{});
+    for (; t < T; ++t) step(MmInt<0>{}, MmInt<0>{}, MmInt<0>{}, MmInt<0>{});
+    if (!grp) mm_barrier();
+    // every fragment has been read: the next tile's first copies land while this one is stored
+    const int em0 = m0, en0 = n0, esp = sp;
+    const bool more = id + stride < last;
+    if (more) {
+      id += stride;
+      begin(id);
+    }
+    // lane l: columns 16 n + 4 (l / 16) .. + 3 of row l % 16
+#pragma unroll
+    for (int m = 0; m < FM; ++m) {
+      const int row = em0 + grp * (BM / 2) + m * 16 + fr, col = en0 + wn * (BN / 4);
+      if (row >= a.M) continue;
+      if constexpr (EPI == kMmGeglu) {
+#pragma unroll
+        for (int n = 0; n < FN; n += 2)
+          if (col + n * 16 < a.N) mm_store_geglu(a, row, (col + n * 16) / 2 + fg * 4, acc[n][m], acc[n + 1][m]);
+      } else {
+#pragma unroll
+        for (int n = 0; n < FN; ++n)
+          if (col + n * 16 < a.N) mm_store<EPI>(a, esp, row, col + n * 16 + fg * 4, acc[n][m]);
+      }
+    }
+    if (!more) return;
+    mm_wait_vm<0>();  // copies and stores (which complete in no order with the copies)
   }
 #endif
 }
@@ -364,7 +404,7 @@ __global__ __launch_bounds__(512 + NP * 64) void mm_pw_kernel(MmArgs a) {
   __shared__ __align__(1024) uint8_t lds[S * kStage];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int m_t, n_t, sp;
-  mm_tile(a, BM, BN, m_t, n_t, sp);
+  mm_tile(a, BM, BN, mm_first(mm_tiles(a, BM, BN)), m_t, n_t, sp);
   const int m0 = m_t * BM, n0 = n_t * BN;
   const int t0 = sp * (a.K / 64) / a.split, T = (sp + 1) * (a.K / 64) / a.split - t0;
   mm_lds* ldsb = (mm_lds*)lds;
@@ -476,6 +516,7 @@ __global__ __launch_bounds__(512 + NP * 64) void mm_pw_kernel(MmArgs a) {
 // ---------------------------------------------------------------------------------------------
 // host: the tiles there are, launches and the choice among them
 // ---------------------------------------------------------------------------------------------
+constexpr unsigned kMmCus = 256;
 enum MmCfg { kMm256x256 = 0, kMm256x192, kMm192x256, kMm128x128, kMm128x96, kMm128x64, kMm64x96, kMm64x64, kMmCfgs };
 constexpr int kMmBm[kMmCfgs] = {256, 256, 192, 128, 128, 128, 64, 64}, kMmBn[kMmCfgs] = {256, 192, 256, 128, 96, 64, 96, 64};
 
@@ -484,15 +525,16 @@ inline bool mm_cfg_has(int cfg, int epi) { return epi != kMmGeglu || (cfg != kMm
 template <int EPI>
 inline bool mm_launch_epi(int cfg, const MmArgs& a, hipStream_t st) {
   const unsigned grid = (unsigned)((a.M + kMmBm[cfg] - 1) / kMmBm[cfg]) * (unsigned)((a.N + kMmBn[cfg] - 1) / kMmBn[cfg]) * (unsigned)a.split;
+  const unsigned pp = grid < kMmCus ? grid : kMmCus;  // mm_pp: one workgroup per CU, which takes tile after tile
   switch (cfg) {
-    case kMm256x256: mm_pp_kernel<8, 4, 2, 3, EPI><<<grid, 512, 0, st>>>(a); break;
-    case kMm192x256: mm_pp_kernel<6, 4, 2, 3, EPI><<<grid, 512, 0, st>>>(a); break;
+    case kMm256x256: mm_pp_kernel<8, 4, 2, 3, EPI><<<pp, 512, 0, st>>>(a); break;
+    case kMm192x256: mm_pp_kernel<6, 4, 2, 3, EPI><<<pp, 512, 0, st>>>(a); break;
     case kMm128x128: mm_pw_kernel<4, 4, 4, 2, EPI><<<grid, 640, 0, st>>>(a); break;
     case kMm128x64: mm_pw_kernel<4, 2, 6, 2, EPI><<<grid, 640, 0, st>>>(a); break;
     case kMm64x64: mm_pw_kernel<2, 2, 5, 2, EPI><<<grid, 640, 0, st>>>(a); break;
     default:
       if constexpr (EPI != kMmGeglu) {
-        if (cfg == kMm256x192) mm_pp_kernel<8, 3, 2, 3, EPI><<<grid, 512, 0, st>>>(a);
+        if (cfg == kMm256x192) mm_pp_kernel<8, 3, 2, 3, EPI><<<pp, 512, 0, st>>>(a);
         else if (cfg == kMm128x96) mm_pw_kernel<4, 3, 5, 2, EPI><<<grid, 640, 0, st>>>(a);
         else if (cfg == kMm64x96) mm_pw_kernel<2, 3, 6, 2, EPI><<<grid, 640, 0, st>>>(a);
         else return false;
