@@ -1021,8 +1021,6 @@ int pi05_prime_prefix(pi05_ctx* c, const void* const* k_layers, const void* cons
   ka.batch = d.batch;
   ka.prefix_len = d.prefix_len;
   ka.s_pad = kv_keys;
-  ka.suffix_base = persistent ? kv_keys : d.prefix_len;
-  HIPCHK(c, launch_prime_kv(ka, d.depth, st));
   PrimeTablesArgs ta{};
   ta.prefix_pad = prefix_pad;
   ta.inv_freq = c->inv_freq;
@@ -1033,7 +1031,7 @@ int pi05_prime_prefix(pi05_ctx* c, const void* const* k_layers, const void* cons
   ta.prefix_len = d.prefix_len;
   ta.s_pad = persistent ? kv_keys + 64 : kv_keys;
   ta.suffix_base = persistent ? kv_keys : d.prefix_len;
-  HIPCHK(c, launch_prime_tables(ta, d.batch, st));
+  HIPCHK(c, launch_prime(ka, ta, d.depth, st));
   c->primed = true;
   return PI05_OK;
 }

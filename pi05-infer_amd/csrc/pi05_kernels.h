@@ -19,8 +19,7 @@ struct PrimeKvArgs {
   int64_t row_stride;    // elements between prefix positions
   u16* kcache;           // [depth][B] fragment-major blocks of s_pad * D
   u16* vcache;
-  int batch, prefix_len, s_pad;
-  int suffix_base;  // keys [suffix_base, suffix_base + A) belong to the action tokens: left untouched
+  int batch, prefix_len, s_pad;  // s_pad: a multiple of 32
 };
 
 struct PrimeTablesArgs {
@@ -210,8 +209,7 @@ int denoise_loop_threads();
 const void* denoise_loop_kernel_ptr(int batch);  // the instance launch_denoise_loop uses for `batch`
 
 hipError_t launch_pack_weight(const void* src, u16* dst, int N, int K, hipStream_t st);
-hipError_t launch_prime_kv(const PrimeKvArgs& a, int depth, hipStream_t st);
-hipError_t launch_prime_tables(const PrimeTablesArgs& a, int batch, hipStream_t st);
+hipError_t launch_prime(const PrimeKvArgs& a, const PrimeTablesArgs& ta, int depth, hipStream_t st);
 hipError_t launch_export_invariants(const ExportInvariantsArgs& a, hipStream_t st);
 hipError_t launch_gemv_rows(const GemvArgs& a, hipStream_t st);
 // temb[s][0:W/2] = sin(2 pi t_s / period_i), temb[s][W/2:W] = cos(...) in float64, rounded to fp32,

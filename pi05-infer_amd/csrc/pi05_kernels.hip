@@ -36,68 +36,97 @@ __global__ void pack_weight_kernel(const u16* __restrict__ src, u16* __restrict_
   }
 }
 
-// Prefix K/V [B, 1, P, D] (strided) -> fragment-major cache keys [0, P); keys [P+A, S_pad) are
-// zeroed so padded lanes never carry NaN/Inf into the masked MFMA products.
-__global__ void prime_kv_kernel(PrimeKvArgs a) {
-  const int layer = blockIdx.z;
-  const int b = blockIdx.y;
-  const u16* ksrc = reinterpret_cast<const u16*>(a.k_ptrs[layer]) + (size_t)b * a.batch_stride;
-  const u16* vsrc = reinterpret_cast<const u16*>(a.v_ptrs[layer]) + (size_t)b * a.batch_stride;
-  u16* kdst = a.kcache + ((size_t)layer * a.batch + b) * a.s_pad * kHeadDim;
-  u16* vdst = a.vcache + ((size_t)layer * a.batch + b) * a.s_pad * kHeadDim;
-  // one thread handles 8 consecutive d of one key
-  const int per_key = kHeadDim / 8;
-  const int total = a.s_pad * per_key;
-  for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
-    const int key = idx / per_key;
-    const int d0 = (idx % per_key) * 8;
-    u16x8 kv8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    u16x8 vv8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    const bool is_prefix = key < a.prefix_len;
-    if (is_prefix) {
-      kv8 = *reinterpret_cast<const u16x8*>(ksrc + (size_t)key * a.row_stride + d0);
-      vv8 = *reinterpret_cast<const u16x8*>(vsrc + (size_t)key * a.row_stride + d0);
-    } else if (key >= a.suffix_base && key < a.suffix_base + kHorizon) {
-      continue;  // action-token keys are written by every step's qkv projection
-    }
-    // K: 8 consecutive d of one key are 8 consecutive elements of one lane
-    *reinterpret_cast<u16x8*>(kdst + kfrag_index(key, d0)) = kv8;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) vdst[vfrag_index(key, d0 + j)] = vv8[j];
-  }
-}
+// Everything a predict's prefix sets up, in one launch.
+//
+// K/V workgroups, one per (layer, sample, 32-key block): prefix K/V [B, 1, P, D] (strided) -> fragment-major
+// cache keys [0, P); the keys behind them are zeroed so padded lanes never carry NaN/Inf into the masked MFMA
+// products (the graph schedule's action-token keys among them, which every step's qkv projection writes
+// before its attention reads them).  Bound by memory: a V fragment's 16 bytes hold 8 keys of one dim, so
+// the block goes through LDS and every store is 16 bytes (2-byte stores straight from the rows took 22.5 us at
+// 18 layers of 968 keys, this 9).
+//
+// Table workgroups, kTabWgs per sample, kTabToks tokens each: positions sum(pad) + t (engine.py:476-477), key-valid
+// mask, bf16 RoPE tables.  Bound by the sines and cosines (one workgroup per sample took 19 us); each
+// workgroup counts the sample's pad for itself.
+constexpr int kTabToks = 4, kTabWgs = (kHorizon + kTabToks - 1) / kTabToks;
 
-// Per batch row: positions sum(pad) + t (engine.py:476-477), key-valid mask, bf16 RoPE tables.
-__global__ void prime_tables_kernel(PrimeTablesArgs a) {
-  const int b = blockIdx.x;
+__device__ __forceinline__ void prime_tables(const PrimeTablesArgs& a, int b, int w) {
   __shared__ int s_cnt[256];
+  const int tid = threadIdx.x;
   const uint8_t* pad = a.prefix_pad + (size_t)b * a.prefix_len;
   int cnt = 0;
-  for (int p = threadIdx.x; p < a.prefix_len; p += blockDim.x) cnt += pad[p] ? 1 : 0;
-  s_cnt[threadIdx.x] = cnt;
+  for (int p = tid; p < a.prefix_len; p += 256) cnt += pad[p] ? 1 : 0;
+  s_cnt[tid] = cnt;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s_cnt[threadIdx.x] += s_cnt[threadIdx.x + w];
+  for (int n = 128; n > 0; n >>= 1) {
+    if (tid < n) s_cnt[tid] += s_cnt[tid + n];
     __syncthreads();
   }
   const int base = s_cnt[0];
   uint8_t* valid = a.valid + (size_t)b * a.s_pad;
-  for (int key = threadIdx.x; key < a.s_pad; key += blockDim.x) {
+  for (int key = w * 256 + tid; key < a.s_pad; key += kTabWgs * 256) {
     uint8_t v = 0;
     if (key < a.prefix_len) v = pad[key] ? 1 : 0;
     else if (key >= a.suffix_base && key < a.suffix_base + kHorizon) v = 1;
     valid[key] = v;
   }
-  for (int idx = threadIdx.x; idx < kHorizon * kHeadDim; idx += blockDim.x) {
-    const int t = idx / kHeadDim;
-    const int d = idx % kHeadDim;
-    const int pos = base + t;
-    if (d == 0) a.positions[b * kHorizon + t] = pos;
-    // emb = cat(freqs, freqs): dims d and d + D/2 share inv_freq[d % (D/2)]
-    const float freq = fmul(a.inv_freq[d % kHalfDim], (float)pos);
-    const size_t o = ((size_t)b * kHorizon + t) * kHeadDim + d;
+  // thread d: dim d of kTabToks tokens; emb = cat(freqs, freqs): dims d and d + D/2 share inv_freq[d % (D/2)]
+  const float inv = a.inv_freq[tid % kHalfDim];
+#pragma unroll
+  for (int i = 0; i < kTabToks; ++i) {
+    const int t = w * kTabToks + i, pos = base + t;
+    if (t >= kHorizon) break;
+    if (tid == 0) a.positions[b * kHorizon + t] = pos;
+    const float freq = fmul(inv, (float)pos);
+    const size_t o = ((size_t)b * kHorizon + t) * kHeadDim + tid;
     a.cos_tab[o] = f2bf(cosf(freq));
     a.sin_tab[o] = f2bf(sinf(freq));
+  }
+}
+
+__global__ __launch_bounds__(256) void prime_kernel(PrimeKvArgs a, PrimeTablesArgs ta) {
+  static_assert(kHeadDim == 256, "one thread per dim");
+  const int tabs = a.batch * kTabWgs;
+  if ((int)blockIdx.x < tabs) {  // the tables first: theirs is the longest chain
+    prime_tables(ta, blockIdx.x / kTabWgs, blockIdx.x % kTabWgs);
+    return;
+  }
+  __shared__ __align__(16) u16 s_v[32][kHeadDim];
+  const int nkb = a.s_pad / 32;
+  int id = blockIdx.x - tabs;
+  const int kb = id % nkb;
+  id /= nkb;
+  const int b = id % a.batch, layer = id / a.batch, tid = threadIdx.x;
+  const u16* ksrc = reinterpret_cast<const u16*>(a.k_ptrs[layer]) + (size_t)b * a.batch_stride;
+  const u16* vsrc = reinterpret_cast<const u16*>(a.v_ptrs[layer]) + (size_t)b * a.batch_stride;
+  const size_t dst = (((size_t)layer * a.batch + b) * a.s_pad + (size_t)kb * 32) * kHeadDim;
+  u16 *kdst = a.kcache + dst, *vdst = a.vcache + dst;
+  // pass i: key i * 8 + tid / 32 of the block, dims 8 (tid % 32) .. + 7
+  const int d0 = (tid & 31) * 8;
+  u16x8 k8[4], v8[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int key = kb * 32 + i * 8 + (tid >> 5);
+    const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    const bool in = key < a.prefix_len;
+    k8[i] = in ? *reinterpret_cast<const u16x8*>(ksrc + (size_t)key * a.row_stride + d0) : zero;
+    v8[i] = in ? *reinterpret_cast<const u16x8*>(vsrc + (size_t)key * a.row_stride + d0) : zero;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 8 + (tid >> 5);
+    // K: 8 consecutive d of one key are 8 consecutive elements of one lane
+    *reinterpret_cast<u16x8*>(kdst + kfrag_index(r, d0)) = k8[i];
+    *reinterpret_cast<u16x8*>(&s_v[r][d0]) = v8[i];
+  }
+  __syncthreads();
+  // pass g: dim tid, the 8 keys vkey(0, g, 0 .. 7) of the block
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    u16x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = s_v[vkey(0, g, j)][tid];
+    *reinterpret_cast<u16x8*>(vdst + vfrag_index(vkey(0, g, 0), tid)) = o;
   }
 }
 
@@ -710,14 +739,8 @@ hipError_t launch_pack_weight(const void* src, u16* dst, int N, int K, hipStream
   return hipGetLastError();
 }
 
-hipError_t launch_prime_kv(const PrimeKvArgs& a, int depth, hipStream_t st) {
-  dim3 grid(32, a.batch, depth);
-  prime_kv_kernel<<<grid, 256, 0, st>>>(a);
-  return hipGetLastError();
-}
-
-hipError_t launch_prime_tables(const PrimeTablesArgs& a, int batch, hipStream_t st) {
-  prime_tables_kernel<<<batch, 256, 0, st>>>(a);
+hipError_t launch_prime(const PrimeKvArgs& a, const PrimeTablesArgs& ta, int depth, hipStream_t st) {
+  prime_kernel<<<a.batch * kTabWgs + depth * a.batch * (a.s_pad / 32), 256, 0, st>>>(a, ta);
   return hipGetLastError();
 }
 

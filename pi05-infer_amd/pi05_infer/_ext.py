@@ -417,7 +417,7 @@ class DenoiseContext:
                     raise ValueError(f"{name}[{i}] shape/strides differ from layer 0")
         pad = prefix_pad
         if pad.dtype == torch.bool:
-            pad = pad.to(torch.uint8)
+            pad = pad.view(torch.uint8)  # the same bytes: no kernel
         if pad.dtype != torch.uint8 or tuple(pad.shape) != (d.batch, d.prefix_len):
             raise ValueError(f"prefix_pad must be bool/uint8 [{d.batch}, {d.prefix_len}]")
         pad = pad.to(self.device).contiguous()
@@ -574,7 +574,7 @@ class PrefixContext:
         if tuple(embeds.shape) != (d.batch, d.prefix_len, d.width):
             raise ValueError(f"embeds shape {tuple(embeds.shape)} != {(d.batch, d.prefix_len, d.width)}")
         ep = _ptr(embeds, torch.bfloat16, "embeds", self.device)
-        pad = prefix_pad.to(torch.uint8) if prefix_pad.dtype == torch.bool else prefix_pad
+        pad = prefix_pad.view(torch.uint8) if prefix_pad.dtype == torch.bool else prefix_pad  # the same bytes: no kernel
         if pad.dtype != torch.uint8 or tuple(pad.shape) != (d.batch, d.prefix_len):
             raise ValueError(f"prefix_pad must be bool/uint8 [{d.batch}, {d.prefix_len}]")
         pad = pad.to(self.device).contiguous()
