@@ -35,9 +35,7 @@ constexpr int kVIp = 4352;
 constexpr int kVGrid = kVImg / kVPatch, kVS = kVGrid * kVGrid;  // 16 x 16 = 256 patches
 constexpr int kVPD = kVC * kVPatch * kVPatch;                   // 588 values per patch
 constexpr int kVQkvN = 3 * kVW;                                 // 3456 fused q|k|v columns
-// attention operands, per (image, head): head dim padded to 96 for Q.K^T (3 k-steps of 32) and to
-// 80 for P.V (5 d-tiles of 16); the padding stays zero
-constexpr int kVKs = 3, kVDt = 5;
+constexpr int kVDt = 5;  // d-tiles of 16 of P.V, the last one half used
 // per-layer packed bf16 weights: [Wq; Wk; Wv] | Wo | W1 | W2; fp32 parameters: bqkv | bo | b1 | b2 |
 // ln1w | ln1b | ln2w | ln2b
 constexpr size_t kVOffQkv = 0, kVOffO = kVOffQkv + (size_t)kVQkvN * kVW, kVOff1 = kVOffO + (size_t)kVW * kVW,
@@ -52,14 +50,11 @@ constexpr int kVLibRows = 1024;
 
 thread_local std::string g_vision_err;
 
-// Attention operands in LDS, per (image, head): K over 96 padded head dims as the A operand of
-// S^T = K Q^T (fragment (key tile, d-step)), V over 80 padded dims as the A operand of
-// O^T = V^T P^T (fragment (key block, d-tile)) with the 32-key permutation vkey, so the P^T operand
-// is the S^T accumulator a lane already holds.  The padding dims are zero.
-constexpr int kVKFrags = (kVS / 16) * kVKs, kVVFrags = (kVS / 32) * kVDt;
-// V fragments in LDS carry 16 bytes of padding after each 16-lane group (a fragment = 4 groups of
-// 272 bytes), so the transposing 2-byte stores of one wave spread over 32 banks
-constexpr int kVVGroup = 136, kVVFrag = 4 * kVVGroup;  // in bf16 elements
+// Attention operands in LDS, per (image, head), rows as they come from the q|k|v product: V rows of 72 head
+// dims, then K rows of 72 dims, 8 zeros (what the third d-step of Q.K^T reads past dim 71) and 8 of padding.
+// Pitches of 144 and 176 bytes spread the 16 rows of a fragment read evenly over the banks, and the whole is 80 KiB:
+// two workgroups a CU.
+constexpr int kVVPitch = kVD, kVKPitch = 88, kVAttnLds = kVS * (kVVPitch + kVKPitch);  // in bf16 elements
 
 // im2col: patches[(n, p)][c*196 + ky*14 + kx] = pixels[n][c][14 py + ky][14 px + kx], p = 16 py + px
 __global__ __launch_bounds__(256) void im2col_kernel(const float* px, float* patches, int n_img) {
@@ -161,117 +156,105 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const u16* x, const u16*
   }
 }
 
-// MHA over one image's 256 patches, straight from the fused q|k|v GEMM output [M, 3456]:
-// workgroup = (image, head, half of the queries), 8 waves (two per SIMD, so one wave's softmax
-// overlaps the other's MFMAs).  The workgroup stages the head's K and V for all 256 keys into LDS
-// in fragment order (16-byte global loads of 8 head dims of one key); wave w loads its query m-tile
-// 8 half + w as B fragments straight from global memory and streams the
-// 8 key blocks of 32 through the online-softmax update: fp32 scores scaled by 72^-0.5 (no bf16
-// rounding of the scores: the reference runs SDPA's flash kernel), P rounded to bf16 for P.V.
-constexpr int kVAttnWaves = 8, kVKPass = (kVS / 16) * kVKs / kVAttnWaves, kVVPass = (kVS / 32) * kVDt / kVAttnWaves;
+// MHA over one image's 256 patches, straight from the fused q|k|v product [M, 3456]: workgroup =
+// (image, head, half of the queries), wave w = query m-tile 8 half + w over all 256 keys.  Scores are fp32
+// (no bf16 rounding of the scores: the reference runs SDPA's flash kernel); all of a query's 256 scores fit
+// the wave's registers, so the softmax is one pass (one maximum, one sum, no rescaling of O), and P is rounded
+// to bf16 for P.V.  S^T = K Q^T leaves a lane the keys 4 (l / 16) .. + 3 of a key tile, which is the P^T operand's
+// order once V's fragments take the same keys: ds_read_b64_tr_b16 reads them transposed from V's rows (lane i of
+// 16 points at 4 dims of key i / 4 and gets dim i of the 4 keys).
+// Bound by latency (a chain of load, LDS, MFMA, exp): two workgroups a CU hide it where there are enough.
+// 1 image 9.9 -> 7.7 us, 24 images 38 -> 25.8 us against the online softmax over V fragments scattered by 2-byte stores.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-__global__ __launch_bounds__(512) void vision_attn_kernel(const u16* qkv, u16* out) {
-  __shared__ __align__(16) u16 s_k[kVKFrags * 512];
-  __shared__ __align__(16) u16 s_v[kVVFrags * kVVFrag];
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void vision_attn_kernel(const u16* qkv, u16* out) {
+#ifdef __HIP_DEVICE_COMPILE__
+  __shared__ __align__(16) u16 s_kv[kVAttnLds];
+  u16 *s_v = s_kv, *s_k = s_kv + kVS * kVVPitch;
   const int half = blockIdx.x & 1, head = (blockIdx.x >> 1) % kVH, n = (blockIdx.x >> 1) / kVH;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, mt = half * kVAttnWaves + wave;
-  const u16* base = qkv + (size_t)n * kVS * kVQkvN + head * kVD;  // row r of the image: q | k | v at +0 | +W | +2W
-  const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  static_assert(kVKPass * kVAttnWaves == (kVS / 16) * kVKs && kVVPass * kVAttnWaves == (kVS / 32) * kVDt, "staging passes");
-  // K: pass (wave, t) fills fragment f = 6 wave + t = (key tile f / 3, d-step f % 3) whole: lane l
-  // loads dims 8 (4 (f % 3) + l / 16) .. +7 of key 16 (f / 3) + l % 16 (zero beyond dim 72) and
-  // stores them at its own 16-byte slot, so each 16-lane store group covers all banks once.
-  // V: pass (wave, t) = combo 5 wave + t = (key block combo / 5, chunk pair combo % 5): lanes 0-31
-  // load the even chunk, lanes 32-63 the odd chunk of the block's 32 keys; element (key r, dim d)
-  // goes to fragment (r / 32, d / 16), group g, lane d % 16, slot j (vkey's inverse).
-  u16x8 kv[kVKPass], vv[kVVPass];  // every global load is issued before the first LDS store
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, mt = half * 8 + wave, r = lane & 15, g = lane >> 4;
+  const u16* base = qkv + (size_t)n * kVS * kVQkvN + head * kVD;  // row i of the image: q | k | v at +0 | +W | +2W
+  constexpr int kChunks = kVS * (kVD / 8), kPass = (kChunks + 511) / 512;  // 16-byte chunks of K (of V)
+  u16x8 kc[kPass], vc[kPass];
 #pragma unroll
-  for (int t = 0; t < kVKPass; ++t) {
-    const int f = wave * kVKPass + t, r = (f / 3) * 16 + (lane & 15), c = (f % 3) * 4 + (lane >> 4);
-    kv[t] = c < 9 ? *reinterpret_cast<const u16x8*>(base + (size_t)r * kVQkvN + kVW + c * 8) : zero;
+  for (int t = 0; t < kPass; ++t) {
+    const int i = t * 512 + tid;
+    if (i < kChunks) {
+      const u16* src = base + (size_t)(i / 9) * kVQkvN + (i % 9) * 8;
+      kc[t] = *reinterpret_cast<const u16x8*>(src + kVW);
+      vc[t] = *reinterpret_cast<const u16x8*>(src + 2 * kVW);
+    }
   }
+  // B operand of S^T: query r, dims 32 ds + 8 g .. + 7 (zero from 72)
+  const u16* qrow = base + (size_t)(mt * 16 + r) * kVQkvN;
+  const bf16x8 q0 = load_frag(qrow + g * 8), q1 = load_frag(qrow + 32 + g * 8);
+  const bf16x8 q2 = g == 0 ? load_frag(qrow + 64) : zero_frag();
 #pragma unroll
-  for (int t = 0; t < kVVPass; ++t) {
-    const int combo = wave * kVVPass + t, r = (combo / 5) * 32 + (lane & 31), c = (combo % 5) * 2 + (lane >> 5);
-    vv[t] = c < 9 ? *reinterpret_cast<const u16x8*>(base + (size_t)r * kVQkvN + 2 * kVW + c * 8) : zero;
+  for (int t = 0; t < kPass; ++t) {
+    const int i = t * 512 + tid;
+    if (i < kChunks) {
+      *reinterpret_cast<u16x8*>(s_k + (i / 9) * kVKPitch + (i % 9) * 8) = kc[t];
+      *reinterpret_cast<u16x8*>(s_v + i * 8) = vc[t];
+    }
   }
-#pragma unroll
-  for (int t = 0; t < kVKPass; ++t) *reinterpret_cast<u16x8*>(s_k + (wave * kVKPass + t) * 512 + lane * 8) = kv[t];
-#pragma unroll
-  for (int t = 0; t < kVVPass; ++t) {
-    const int combo = wave * kVVPass + t, r = lane & 31, c = (combo % 5) * 2 + (lane >> 5);
-    const int g = (r & 15) >> 2, j = r < 16 ? (r & 3) : 4 + (r & 3);
-    u16* dst = s_v + ((combo / 5) * kVDt + (c >> 1)) * kVVFrag + g * kVVGroup + (c & 1) * 64 + j;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) dst[e * 8] = vv[t][e];
-  }
-  bf16x8 q[kVKs];
-  const u16* qrow = base + (size_t)(mt * 16 + (lane & 15)) * kVQkvN;
-#pragma unroll
-  for (int ds = 0; ds < kVKs; ++ds) {
-    const int d = ds * 32 + (lane >> 4) * 8;
-    q[ds] = d < kVD ? load_frag(qrow + d) : zero_frag();
-  }
+  if (tid < kVS) *reinterpret_cast<u16x8*>(s_k + tid * kVKPitch + kVD) = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
   __syncthreads();
-  const float scale = 0.11785113019775793f;  // 72 ** -0.5
-  float m_run = -INFINITY, l_run = 0.f;
-  f32x4 oacc[kVDt];
+  f32x4 s[kVS / 16];
 #pragma unroll
-  for (int d = 0; d < kVDt; ++d) oacc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int blk = 0; blk < kVS / 32; ++blk) {
-    bf16x8 k[2 * kVKs], v[kVDt];
+  for (int kt = 0; kt < kVS / 16; ++kt) {
+    const u16* k = s_k + (kt * 16 + r) * kVKPitch;
+    f32x4 acc = mfma16x16x32(load_frag(k + g * 8), q0, f32x4{0.f, 0.f, 0.f, 0.f});
+    acc = mfma16x16x32(load_frag(k + 32 + g * 8), q1, acc);
+    s[kt] = mfma16x16x32(load_frag(k + (g == 0 ? 64 : kVD)), q2, acc);  // every group past the row's end: its zeros
+  }
+  float m = s[0][0];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+  for (int kt = 0; kt < kVS / 16; ++kt)
 #pragma unroll
-      for (int ds = 0; ds < kVKs; ++ds) k[t * kVKs + ds] = load_frag(s_k + ((2 * blk + t) * kVKs + ds) * 512 + lane * 8);
+    for (int i = 0; i < 4; ++i) m = fmaxf(m, s[kt][i]);
+  m = lane_max_xor32(lane_max_xor16(m));
+  // exp((s - m) 72^-0.5) as exp2
+  const float c = 0.11785113019775793f * 1.4426950408889634f;
+  float l = 0.f;
+  bf16x8 p[kVS / 32];
 #pragma unroll
-    for (int dt = 0; dt < kVDt; ++dt) v[dt] = load_frag(s_v + (blk * kVDt + dt) * kVVFrag + (lane >> 4) * kVVGroup + (lane & 15) * 8);
-    f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int ds = 0; ds < kVKs; ++ds)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) sacc[t] = mfma16x16x32(k[t * kVKs + ds], q[ds], sacc[t]);
-    float s[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s[i] = sacc[0][i] * scale;
-      s[4 + i] = sacc[1][i] * scale;
-    }
-    float bm = s[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) bm = fmaxf(bm, s[i]);
-    bm = fmaxf(bm, __shfl_xor(bm, 16));
-    bm = fmaxf(bm, __shfl_xor(bm, 32));
-    const float m_new = fmaxf(m_run, bm);
-    const float alpha = __expf(m_run - m_new);  // m_run = -inf on the first block: alpha = 0
-    float e[8], esum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      e[i] = __expf(s[i] - m_new);
-      esum += e[i];
-    }
-    l_run = l_run * alpha + esum;
-    m_run = m_new;
+  for (int kb = 0; kb < kVS / 32; ++kb) {
     u16x8 pf;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) pf[i] = f2bf(e[i]);
-    const bf16x8 pfrag = as_bf16x8(pf);
-#pragma unroll
-    for (int dt = 0; dt < kVDt; ++dt) oacc[dt] = mfma16x16x32(v[dt], pfrag, oacc[dt] * alpha);
+    for (int j = 0; j < 8; ++j) {
+      const float e = __builtin_amdgcn_exp2f((s[2 * kb + j / 4][j % 4] - m) * c);
+      l += e;
+      pf[j] = f2bf(e);
+    }
+    p[kb] = as_bf16x8(pf);
   }
-  float l = l_run;
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l = lane_sum_xor32(lane_sum_xor16(l));
   const float inv = 1.0f / l;
-  const int tok = mt * 16 + (lane & 15), g = lane >> 4;
-  u16* orow = out + ((size_t)n * kVS + tok) * kVW + head * kVD;
+  // A operand of O^T = V^T P^T: keys 4 g .. + 3 and 16 + 4 g .. + 3 of block kb, dim 16 dt + r (dims past 71 read
+  // what follows the row; their rows of O^T are not stored)
+  const u16* vl = s_v + (4 * g + (r >> 2)) * kVVPitch + (r & 3) * 4;
+  f32x4 o[kVDt];
+#pragma unroll
+  for (int dt = 0; dt < kVDt; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kb = 0; kb < kVS / 32; ++kb)
+#pragma unroll
+    for (int dt = 0; dt < kVDt; ++dt) {
+      const u16* v = vl + kb * 32 * kVVPitch + dt * 16;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)v);
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(v + 16 * kVVPitch));
+      u16x8 f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = (u16)lo[j], f[4 + j] = (u16)hi[j];
+      o[dt] = mfma16x16x32(as_bf16x8(f), p[kb], o[dt]);
+    }
+  u16* orow = out + ((size_t)n * kVS + mt * 16 + r) * kVW + head * kVD + g * 4;
 #pragma unroll
   for (int dt = 0; dt < kVDt; ++dt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = dt * 16 + g * 4 + i;
-      if (d < kVD) orow[d] = f2bf(oacc[dt][i] * inv);
-    }
+    if (dt * 16 + g * 4 < kVD)
+      *reinterpret_cast<u16x4*>(orow + dt * 16) = u16x4{f2bf(o[dt][0] * inv), f2bf(o[dt][1] * inv), f2bf(o[dt][2] * inv), f2bf(o[dt][3] * inv)};
+#endif
 }
 
 __global__ __launch_bounds__(256) void scale_kernel(u16* x, size_t total, float s) {
