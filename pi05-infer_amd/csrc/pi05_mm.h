@@ -566,6 +566,14 @@ inline bool mm_launch(int cfg, int epi, const MmArgs& a, hipStream_t st) {
   }
 }
 
+// Holds the stream for `ticks` of the 100 MHz counter (or the bounded number of polls).
+static __global__ void mm_hold_kernel(unsigned ticks) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+  for (int i = 0; i < 1 << 16 && __builtin_amdgcn_s_memrealtime() - t0 < ticks; ++i) __builtin_amdgcn_s_sleep(2);
+#endif
+}
+
 // The tile and the K split of one product.
 struct MmPlan {
   int cfg = -1, split = 1;
@@ -575,10 +583,12 @@ struct MmPlan {
 // The fastest tile and K split for a product: every tile with every split in [smin, smax] that leaves a split
 // at least 4 k-tiles, timed on the caller's buffers as the layer loop runs them (run r reads the weights at
 // a.W + (r mod w_count) * w_stride bytes, so they stream from memory; values do not affect the choice of
-// path), the 4 fastest again in 3 interleaved rounds.  Timed rather than computed from the sizes because two effects
-// of equal size decide: how evenly the tiles fill 256 CUs (M = 768, N = 4304: 128 x 128 12.6 us, 128 x 96
-// 19.6 us) and the copies per MFMA (M = 968, N = 32768: 256 x 256 115 us, 128 x 128 166 us).  split_ms: what
-// the reader of the partial sums pays per split.
+// path), the 6 fastest again in 4 interleaved rounds of 20 runs.  The stream is held while the host
+// enqueues the runs: a 6 us product is otherwise timed at the rate the host launches it, where all tiles look
+// alike (the picks of a 256-row layer then changed from context to context).  Timed rather than computed
+// from the sizes because two effects of equal size decide: how evenly the tiles fill 256 CUs (M = 768, N =
+// 4304: 128 x 128 12.6 us, 128 x 96 19.6 us) and the copies per MFMA (M = 968, N = 32768: 256 x 256 115 us,
+// 128 x 128 166 us).  split_ms: what the reader of the partial sums pays per split.
 inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_t w_stride, int w_count, hipStream_t st, MmPlan* out) {
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess) return false;
@@ -590,7 +600,9 @@ inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_
   auto time = [&](const MmPlan& c, int reps, float* ms) {
     a.split = c.split;
     a.W = w;
-    bool ok = mm_launch(c.cfg, epi, a, st) && hipEventRecord(e0, st) == hipSuccess;
+    bool ok = mm_launch(c.cfg, epi, a, st);
+    mm_hold_kernel<<<1, 1, 0, st>>>(1500u * (unsigned)reps);  // 15 us a run
+    ok = ok && hipEventRecord(e0, st) == hipSuccess;
     for (int r = 0; r < reps && ok; ++r) {
       a.W = w + (size_t)(r % w_count) * (w_stride / 2);
       ok = mm_launch(c.cfg, epi, a, st);
@@ -601,22 +613,26 @@ inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_
   };
   std::vector<std::pair<float, MmPlan>> c;
   bool ok = true;
+  MmPlan warm;
+  warm.cfg = kMm128x128, warm.split = smin;
+  float ms0 = 0.f;
+  ok = time(warm, 40, &ms0);  // the clock ramps up here
   for (int cfg = 0; cfg < kMmCfgs && ok; ++cfg)
     for (int s = smin; s <= smax && ok; ++s) {
       MmPlan p;
       p.cfg = cfg, p.split = a.split = s;
       a.W = w;
       if (!mm_fits(cfg, epi, a) || (s > 1 && a.K / 64 / s < 4)) continue;
-      ok = time(p, 2, &p.ms);
+      ok = time(p, 6, &p.ms);
       c.emplace_back(p.ms + split_ms * (float)s, p);
     }
   std::sort(c.begin(), c.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-  const size_t n = c.size() < 4 ? c.size() : 4;
+  const size_t n = c.size() < 6 ? c.size() : 6;
   for (size_t i = 0; i < n; ++i) c[i].second.ms = 1e30f;
-  for (int round = 0; round < 3 && ok; ++round)
+  for (int round = 0; round < 4 && ok; ++round)
     for (size_t i = 0; i < n && ok; ++i) {
       float ms = 0.f;
-      ok = time(c[i].second, 10, &ms);
+      ok = time(c[i].second, 20, &ms);
       c[i].second.ms = std::min(c[i].second.ms, ms);
     }
   (void)hipEventDestroy(e0);
