@@ -2,8 +2,8 @@
 //
 // C[M, N] (row-major) = A[M, K] (row-major) . W[N, K]^T (nn.Linear layout), fp32 accumulation.
 // In hipBLASLt's column-major terms that is C^T (N x M) = W (stored K x N, transposed) . A^T
-// (stored K x M).  Options: an fp32 bias per output column added before the one rounding
-// (HIPBLASLT_EPILOGUE_BIAS; the pointer is set per call), fp32 operands, split-K batches.
+// (stored K x M).  bf16 operands and output; option: an fp32 bias per output column added before the one rounding
+// (HIPBLASLT_EPILOGUE_BIAS; the pointer is set per call).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -32,24 +32,19 @@ constexpr int kGemmCandidates = 256;
 inline bool lt_ok(hipblasStatus_t s) { return s == HIPBLAS_STATUS_SUCCESS; }
 
 struct GemmOpts {
-  int batch = 1;                // > 1: split-K over `batch` K-slices of width K of rows ld_k long
-  int ld_k = 0;                 // row length of the A and W operands (0: K)
-  hipDataType ab = HIP_R_16BF;  // operand type (HIP_R_32F for an fp32 GEMM)
-  hipDataType c = HIP_R_16BF;   // output type (split-K partials: HIP_R_32F)
-  bool bias = false;            // fp32 per-column bias before the rounding
-  int ld_c = 0;                 // row length of the output (0: N)
+  int ld_k = 0;       // row length of the A and W operands (0: K)
+  bool bias = false;  // fp32 per-column bias before the rounding
 };
 
 inline bool make_plan(hipblasLtHandle_t h, int M, int N, int K, size_t ws_max, GemmPlan* p, std::string* err, GemmOpts o = GemmOpts{}) {
   const int ld_k = o.ld_k ? o.ld_k : K;
   p->M = M, p->N = N, p->K = K, p->bias = o.bias;
   const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
-  const hipDataType ct = o.batch > 1 ? HIP_R_32F : o.c;
   if (!lt_ok(hipblasLtMatmulDescCreate(&p->desc, HIPBLAS_COMPUTE_32F, HIP_R_32F)) ||
       !lt_ok(hipblasLtMatmulDescSetAttribute(p->desc, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta))) ||
       !lt_ok(hipblasLtMatmulDescSetAttribute(p->desc, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb))) ||
-      !lt_ok(hipblasLtMatrixLayoutCreate(&p->lw, o.ab, K, N, ld_k)) || !lt_ok(hipblasLtMatrixLayoutCreate(&p->la, o.ab, K, M, ld_k)) ||
-      !lt_ok(hipblasLtMatrixLayoutCreate(&p->lc, ct, N, M, o.ld_c ? o.ld_c : N))) {
+      !lt_ok(hipblasLtMatrixLayoutCreate(&p->lw, HIP_R_16BF, K, N, ld_k)) || !lt_ok(hipblasLtMatrixLayoutCreate(&p->la, HIP_R_16BF, K, M, ld_k)) ||
+      !lt_ok(hipblasLtMatrixLayoutCreate(&p->lc, HIP_R_16BF, N, M, N))) {
     *err = "hipBLASLt descriptor creation failed";
     return false;
   }
@@ -60,18 +55,6 @@ inline bool make_plan(hipblasLtHandle_t h, int M, int N, int K, size_t ws_max, G
         !lt_ok(hipblasLtMatmulDescSetAttribute(p->desc, HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &bt, sizeof(bt)))) {
       *err = "hipBLASLt bias epilogue failed";
       return false;
-    }
-  }
-  if (o.batch > 1) {
-    const int32_t bc = o.batch;
-    const int64_t sk = K, sc = (int64_t)(o.ld_c ? o.ld_c : N) * M;
-    for (hipblasLtMatrixLayout_t l : {p->lw, p->la, p->lc}) {
-      const int64_t st = l == p->lc ? sc : sk;
-      if (!lt_ok(hipblasLtMatrixLayoutSetAttribute(l, HIPBLASLT_MATRIX_LAYOUT_BATCH_COUNT, &bc, sizeof(bc))) ||
-          !lt_ok(hipblasLtMatrixLayoutSetAttribute(l, HIPBLASLT_MATRIX_LAYOUT_STRIDED_BATCH_OFFSET, &st, sizeof(st)))) {
-        *err = "hipBLASLt batch layout failed";
-        return false;
-      }
     }
   }
   hipblasLtMatmulPreference_t pref = nullptr;
@@ -92,10 +75,8 @@ inline bool make_plan(hipblasLtHandle_t h, int M, int N, int K, size_t ws_max, G
       seen.push_back(hipblaslt_ext::getIndexFromAlgo(res[i].algo));
     }
   // every other solution the library holds for this problem type that accepts this problem
-  // (split-K / stream-K variants the heuristic leaves out fill the GPU at small M x N)
   std::vector<hipblasLtMatmulHeuristicResult_t> all;
-  const hipDataType ct_all = ct;
-  if (lt_ok(hipblaslt_ext::getAllAlgos(h, hipblaslt_ext::GemmType::HIPBLASLT_GEMM, ta, tb, o.ab, o.ab, ct_all, ct_all, HIPBLAS_COMPUTE_32F, all))) {
+  if (lt_ok(hipblaslt_ext::getAllAlgos(h, hipblaslt_ext::GemmType::HIPBLASLT_GEMM, ta, tb, HIP_R_16BF, HIP_R_16BF, HIP_R_16BF, HIP_R_16BF, HIPBLAS_COMPUTE_32F, all))) {
     const float alpha = 1.f, beta = 0.f;
     for (auto& r : all) {
       const int idx = hipblaslt_ext::getIndexFromAlgo(r.algo);

@@ -1,7 +1,6 @@
 // The pi0.5 vision tower on gfx950: SigLIP So400m/14 + PaliGemma's projector (get_image_features,
 // gemma_pytorch.py:106-107; the tower itself is transformers' SiglipVisionModel).  Per image:
-//   patches (fp32 im2col) . Wpatch^T          hipBLASLt fp32 GEMM
-//   h = bf16(conv + bpatch + pos)              embed_kernel
+//   h = bf16(conv + bpatch + pos)              patch_embed_kernel (fp32 MFMA straight from the pixels)
 //   27 x [ n = LN1(h); q|k|v = n.W^T + b      product (bias epilogue)
 //          attention, 16 heads of 72          vision_attn_kernel (MFMA, K/V staged in LDS)
 //          h = bf16(h + o.Wo^T + bo); n = LN2 product (split-K when faster) + layernorm_kernel
@@ -56,24 +55,95 @@ thread_local std::string g_vision_err;
 // two workgroups a CU.
 constexpr int kVVPitch = kVD, kVKPitch = 88, kVAttnLds = kVS * (kVVPitch + kVKPitch);  // in bf16 elements
 
-// im2col: patches[(n, p)][c*196 + ky*14 + kx] = pixels[n][c][14 py + ky][14 px + kx], p = 16 py + px
-__global__ __launch_bounds__(256) void im2col_kernel(const float* px, float* patches, int n_img) {
-  const size_t total = (size_t)n_img * kVS * kVPD;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-    const size_t row = i / kVPD;
-    const int col = (int)(i % kVPD), n = (int)(row / kVS), p = (int)(row % kVS);
-    const int c = col / (kVPatch * kVPatch), ky = (col / kVPatch) % kVPatch, kx = col % kVPatch;
-    const int y = (p / kVGrid) * kVPatch + ky, x = (p % kVGrid) * kVPatch + kx;
-    patches[i] = px[(((size_t)n * kVC + c) * kVImg + y) * kVImg + x];
-  }
+// h = bf16(conv + patch bias + position embedding) (SiglipVisionEmbeddings, fp32 until here), the 14 x 14 patch
+// convolution as an fp32 MFMA product straight from the pixels: h[(n, 16 py + px)][o] sums pixels[n][c][14 py +
+// ky][14 px + kx] W[o][c 196 + ky 14 + kx], W packed by pack_patch_kernel (1 KiB a wave load: 64-byte pieces of W's
+// own rows took four times as long to load).  Workgroup = 64 output channels, one 16-channel tile a wave, for every
+// stride-th patch row of 16 patches: its weights stay in registers, and a patch row's pixels (14 whole image rows a
+// channel, contiguous) go to LDS as they are, the next patch row's while this one is multiplied.  Lane l holds
+// four consecutive k of channel l % 16, so the four MFMAs of a 16-wide step take k = 16 S + 4 (l / 16) + j; s_off
+// gives the LDS offset of each k within a patch.  Bound by the fp32 matrix rate (157 TFLOP/s: 2.2 us an image).
+// Against im2col, a library product and an embedding pass (us): 1 image 21 -> 13, 3 images 28 -> 20, 24 images 104 -> 98.
+constexpr int kVSteps = (kVPD + 15) / 16, kVRowPix = kVPatch * kVImg;  // 37 steps; 3136 pixels of a patch row and channel
+
+// wp[o / 16][k / 16][lane][4]: lane l holds k = 16 s + 4 (l / 16) .. + 3 of channel l % 16, zeros from k = 588
+__global__ __launch_bounds__(256) void pack_patch_kernel(const float* w, float* wp) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= kVW / 16 * kVSteps * 256) return;
+  const int j = i & 3, l = (i >> 2) & 63, s = (i >> 8) % kVSteps, ot = (i >> 8) / kVSteps, k = s * 16 + (l >> 4) * 4 + j;
+  wp[i] = k < kVPD ? w[(size_t)(ot * 16 + (l & 15)) * kVPD + k] : 0.f;
 }
 
-// h = bf16(conv + patch bias + position embedding) (SiglipVisionEmbeddings, fp32 until here)
-__global__ __launch_bounds__(256) void embed_kernel(const float* conv, const float* pb, const float* pos, u16* h, size_t total) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-    const int c = (int)(i % kVW), p = (int)((i / kVW) % kVS);
-    h[i] = f2bf(conv[i] + pb[c] + pos[(size_t)p * kVW + c]);
+__global__ __launch_bounds__(256) void patch_embed_kernel(const float* px, const float* w, const float* pb, const float* pos, u16* h,
+                                                          int rows, int stride) {
+#ifdef __HIP_DEVICE_COMPILE__
+  // two arrays, not one of two: the compiler then knows that a copy into the one leaves the other alone
+  __shared__ __align__(16) float s_pa[kVC * kVRowPix], s_pb[kVC * kVRowPix];
+  __shared__ __align__(16) uint16_t s_off[kVSteps * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+  constexpr int kNt = kVW / 64;
+  const int o0 = ((int)blockIdx.x % kNt) * 64 + wave * 16;
+  const bool vec = reinterpret_cast<uintptr_t>(px) % 16 == 0;  // a patch row's pixels are 12544 bytes: aligned as px is
+  auto stage = [&](int row, float* buf) {  // patch row `row` (16 an image)
+    const float* src = px + ((size_t)(row / kVGrid) * kVC * kVImg + (row % kVGrid) * kVPatch) * kVImg;
+    if (vec) {
+#pragma unroll
+      for (int c = 0; c < kVC; ++c)
+#pragma unroll
+        for (int i = 0; i < (kVRowPix + 1023) / 1024; ++i) {
+          const int at = i * 1024 + wave * 256;
+          if (at + lane * 4 < kVRowPix)
+            __builtin_amdgcn_global_load_lds(const_cast<float*>(src) + (size_t)c * kVImg * kVImg + at + lane * 4,
+                                             (__attribute__((address_space(3))) float*)buf + c * kVRowPix + at, 16, 0, 0);
+        }
+    } else {
+      for (int c = 0; c < kVC; ++c)
+        for (int i = tid; i < kVRowPix; i += 256) buf[c * kVRowPix + i] = src[(size_t)c * kVImg * kVImg + i];
+    }
+  };
+  int row = (int)blockIdx.x / kNt;
+  stage(row, s_pa);
+  f32x4 wf[kVSteps];
+  const float* wr = w + (size_t)(o0 / 16) * kVSteps * 256 + lane * 4;
+#pragma unroll
+  for (int s = 0; s < kVSteps; ++s) wf[s] = *reinterpret_cast<const f32x4*>(wr + s * 256);
+  for (int k = tid; k < kVSteps * 16; k += 256) {
+    const int c = k / (kVPatch * kVPatch), ky = k / kVPatch % kVPatch;
+    s_off[k] = (uint16_t)(k < kVPD ? c * kVRowPix + ky * kVImg + k % kVPatch : 0);
   }
+  const int o = o0 + g * 4;
+  const f32x4 bias = *reinterpret_cast<const f32x4*>(pb + o);
+  auto patch_row = [&](float* cur, float* other) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies of the patch row
+    __syncthreads();                                  // every wave's; and the other buffer is no longer read
+    if (row + stride < rows) stage(row + stride, other);
+    const float* pr = cur + r * kVPatch;
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int s = 0; s < kVSteps; ++s) {
+      const u16x4 off = *reinterpret_cast<const u16x4*>(s_off + s * 16 + g * 4);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {  // an even k and the next one are neighbours in a patch's row (14 is even)
+        float2 v = *reinterpret_cast<const float2*>(pr + off[2 * p]);
+        if (s * 16 + 16 > kVPD && s * 16 + g * 4 >= kVPD) v = float2{0.f, 0.f};
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[s][2 * p], v.x, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[s][2 * p + 1], v.y, acc[1], 0, 0, 0);
+      }
+    }
+    // lane l: channels o0 + 4 (l / 16) .. + 3 of patch l % 16
+    const int t = row * kVGrid + r;
+    const f32x4 ps = *reinterpret_cast<const f32x4*>(pos + (size_t)(t % kVS) * kVW + o);
+    u16x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = f2bf(fadd(fadd(fadd(acc[0][i], acc[1][i]), bias[i]), ps[i]));
+    *reinterpret_cast<u16x4*>(h + (size_t)t * kVW + o) = v;
+    row += stride;
+  };
+  while (row < rows) {
+    patch_row(s_pa, s_pb);
+    if (row < rows) patch_row(s_pb, s_pa);
+  }
+#endif
 }
 
 // h = bf16(x + y), n = bf16((h - mean) / sqrt(var + eps) * w + b) with fp32 statistics
@@ -271,8 +341,8 @@ struct VLayerBind {
 
 struct VisionPlan {
   int L = 0, N = 0, M = 0;
-  size_t w, par, head, h, qkv, act, part, patches, conv, ws;
-  size_t total() const { return w + par + head + 4 * h + qkv + act + part + patches + conv + ws + 16 * 256; }
+  size_t w, par, head, h, qkv, act, part, ws;
+  size_t total() const { return w + par + head + 4 * h + qkv + act + part + ws + 16 * 256; }
 };
 
 size_t vrup(size_t x) { return (x + 255) / 256 * 256; }
@@ -283,14 +353,12 @@ VisionPlan vplan_of(const pi05_vision_dims& d) {
   const size_t M = p.M;
   p.w = vrup((size_t)p.L * kVLayerElems * 2);
   p.par = vrup((size_t)p.L * kVLayerParams * 4);
-  // heads: patch_w [W, 588] + patch_b + pos [256, W] + post w/b (fp32), proj_w bf16, proj_b fp32
-  p.head = vrup(((size_t)kVW * kVPD + kVW + (size_t)kVS * kVW + 2 * kVW + kVProj) * 4 + (size_t)kVProj * kVW * 2);
+  // heads: packed patch_w + patch_b + pos [256, W] + post w/b (fp32), proj_w bf16, proj_b fp32
+  p.head = vrup(((size_t)kVW * kVSteps * 16 + kVW + (size_t)kVS * kVW + 2 * kVW + kVProj) * 4 + (size_t)kVProj * kVW * 2);
   p.h = vrup(M * kVW * 2);
   p.qkv = vrup(M * kVQkvN * 2);
   p.part = vrup((size_t)kVMaxSplits * M * kVW * 4);
   p.act = vrup(M * kVIp * 2);
-  p.patches = vrup(M * kVPD * 4);
-  p.conv = vrup(M * kVW * 4);
   p.ws = kVWorkspace;
   return p;
 }
@@ -337,11 +405,11 @@ struct pi05_vision_ctx {
   char* base = nullptr;
   u16 *w = nullptr, *h = nullptr, *n = nullptr, *y = nullptr, *attn = nullptr, *qkv = nullptr, *act = nullptr, *proj_w = nullptr;
   float *par = nullptr, *patch_w = nullptr, *patch_b = nullptr, *pos = nullptr, *post_w = nullptr, *post_b = nullptr, *proj_b = nullptr,
-        *part = nullptr, *patches = nullptr, *conv = nullptr;
+        *part = nullptr;
   void* ws = nullptr;
   hipblasLtHandle_t lt = nullptr;
   // the bf16 products: on pi05_mm.h, or (from kVLibRows rows, where it measured faster) on hipBLASLt
-  GemmPlan g_patch, g_qkv, g_o, g_fc2, g_proj;
+  GemmPlan g_qkv, g_o, g_fc2, g_proj;
   MmPlan m_qkv, m_o, m_fc1, m_fc2, m_proj;
   bool lib_qkv = false, lib_o = false, lib_fc2 = false, lib_proj = false;
 };
@@ -421,7 +489,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   c->par = reinterpret_cast<float*>(take(p.par));
   char* hd = take(p.head);
   c->patch_w = reinterpret_cast<float*>(hd);
-  c->patch_b = c->patch_w + (size_t)kVW * kVPD;
+  c->patch_b = c->patch_w + (size_t)kVW * kVSteps * 16;
   c->pos = c->patch_b + kVW;
   c->post_w = c->pos + (size_t)kVS * kVW;
   c->post_b = c->post_w + kVW;
@@ -434,8 +502,6 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   c->qkv = reinterpret_cast<u16*>(take(p.qkv));
   c->act = reinterpret_cast<u16*>(take(p.act));
   c->part = reinterpret_cast<float*>(take(p.part));
-  c->patches = reinterpret_cast<float*>(take(p.patches));
-  c->conv = reinterpret_cast<float*>(take(p.conv));
   c->ws = take(p.ws);
   // zeroed once: tuning reads defined data
   e = hipMemset(c->base, 0, p.total());
@@ -446,17 +512,14 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   }
   std::string perr;
   const int M = p.M;
-  GemmOpts f32;
-  f32.ab = HIP_R_32F;
-  f32.c = HIP_R_32F;
   GemmOpts bias;
   bias.bias = true;
   GemmOpts fc2o = bias;
   fc2o.ld_k = kVIp;
   const bool lib = M > kVLibRows;
-  bool ok = lt_ok(hipblasLtCreate(&c->lt)) && make_plan(c->lt, M, kVW, kVPD, kVWorkspace, &c->g_patch, &perr, f32) &&
-            (!lib || (make_plan(c->lt, M, kVQkvN, kVW, kVWorkspace, &c->g_qkv, &perr, bias) && make_plan(c->lt, M, kVW, kVW, kVWorkspace, &c->g_o, &perr, bias) &&
-                      make_plan(c->lt, M, kVW, kVIp, kVWorkspace, &c->g_fc2, &perr, fc2o) && make_plan(c->lt, M, kVProj, kVW, kVWorkspace, &c->g_proj, &perr, bias)));
+  bool ok = !lib || (lt_ok(hipblasLtCreate(&c->lt)) && make_plan(c->lt, M, kVQkvN, kVW, kVWorkspace, &c->g_qkv, &perr, bias) &&
+                     make_plan(c->lt, M, kVW, kVW, kVWorkspace, &c->g_o, &perr, bias) && make_plan(c->lt, M, kVW, kVIp, kVWorkspace, &c->g_fc2, &perr, fc2o) &&
+                     make_plan(c->lt, M, kVProj, kVW, kVWorkspace, &c->g_proj, &perr, bias));
   if (ok) {
     const float* bz = c->par;  // any fp32 vector long enough (zeros) stands in for the biases while timing
     // (weights rotate over the layers' blocks while timing, as the layer loop streams them)
@@ -465,8 +528,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
     // what a reader of fp32 partials pays per split: 4 bytes per output element at ~4 TB/s, less the
     // bf16 output it would read and the product write otherwise
     const float part_ms = (float)(4.0 * M * kVW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kVW / 4e12 * 1e3);
-    ok = tune_plan(c->lt, &c->g_patch, c->patch_w, c->patches, c->conv, c->ws, nullptr) &&
-         mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+    ok = mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
          mm_tune({c->n, c->w, c->act, bz, M, kVI, kVW, kVW, kVW, kVIp, 1}, kMmGelu, 1, 1, 0.f, ls, nl, nullptr, &c->m_fc1) &&
          mm_tune({c->n, c->proj_w, c->act, bz, M, kVProj, kVW, kVW, kVW, kVProj, 1}, kMmBf16, 1, 1, 0.f, 0, 1, nullptr, &c->m_proj);
     // out_proj and fc2: one product with its bias, or fp32 K splits that the LayerNorm adds
@@ -503,7 +565,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
 
 int pi05_vision_destroy(pi05_vision_ctx* c) {
   if (!c) return PI05_OK;
-  for (GemmPlan* g : {&c->g_patch, &c->g_qkv, &c->g_o, &c->g_fc2, &c->g_proj})
+  for (GemmPlan* g : {&c->g_qkv, &c->g_o, &c->g_fc2, &c->g_proj})
     free_plan(g);
   if (c->lt) hipblasLtDestroy(c->lt);
   if (c->base) hipFree(c->base);
@@ -575,7 +637,7 @@ int pi05_vision_refresh_weights(pi05_vision_ctx* c, void* stream) {
     to_f32(b.p[14], pr + kVPOffLn2w, kVW);
     to_f32(b.p[15], pr + kVPOffLn2b, kVW);
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(c->patch_w, c->b_patch_w, (size_t)kVW * kVPD * 4, k, st);
+  if (e == hipSuccess) pack_patch_kernel<<<kVW / 16 * kVSteps, 256, 0, st>>>(c->b_patch_w, c->patch_w);
   if (e == hipSuccess) e = hipMemcpyAsync(c->patch_b, c->b_patch_b, kVW * 4, k, st);
   if (e == hipSuccess) e = hipMemcpyAsync(c->pos, c->b_pos, (size_t)kVS * kVW * 4, k, st);
   if (e == hipSuccess) e = hipMemcpyAsync(c->proj_w, c->b_proj_w, (size_t)kVProj * kVW * 2, k, st);
@@ -600,9 +662,9 @@ int pi05_vision_forward(pi05_vision_ctx* c, const float* pixels, void* out, void
   const float eps = c->d.ln_eps;
   const size_t M = p.M;
   int rc;
-  im2col_kernel<<<grid_for(M * kVPD), 256, 0, st>>>(pixels, c->patches, p.N);
-  if ((rc = vgemm(c, c->g_patch, c->patch_w, c->patches, c->conv, nullptr, st)) != PI05_OK) return rc;
-  embed_kernel<<<grid_for(M * kVW), 256, 0, st>>>(c->conv, c->patch_b, c->pos, c->h, M * kVW);
+  // two workgroups a CU (their LDS): 28 x 18, the patch rows dealt out evenly
+  const int rows = p.N * kVGrid, each = (rows + 27) / 28, stride = (rows + each - 1) / each;
+  patch_embed_kernel<<<(unsigned)(stride * (kVW / 64)), 256, 0, st>>>(pixels, c->patch_w, c->patch_b, c->pos, c->h, rows, stride);
   const float* pr0 = c->par;
   const unsigned ln_grid = (unsigned)((M + 3) / 4);
   const size_t pstride = M * kVW;
