@@ -57,8 +57,8 @@ thread_local std::string g_prefix_err;
 // ---------------------------------------------------------------------------------------------
 // positions cumsum(pad) - 1 and key-valid bytes of one sample (one workgroup per sample)
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void positions_kernel(const uint8_t* pad, int P, int s_pad, int* pos, uint8_t* valid) {
-  const int b = blockIdx.x, t = threadIdx.x;
+__device__ __forceinline__ void positions(int b, const uint8_t* pad, int P, int s_pad, int* pos, uint8_t* valid) {
+  const int t = threadIdx.x;
   __shared__ int s_cnt[256];
   const uint8_t* pb = pad + (size_t)b * P;
   const int per = (P + 255) / 256, p0 = t * per, p1 = p0 + per < P ? p0 + per : P;
@@ -88,9 +88,9 @@ __global__ __launch_bounds__(256) void positions_kernel(const uint8_t* pad, int 
 // the bf16 rounding of the sum of nsplit fp32 split-K partials ys[s * split_stride + ...], added
 // in split order (the GEMM's own rounding of its full sum).
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const u16* x, const u16* y, const float* w, u16* h_out, u16* n_out, float eps,
-                                                      const float* ys = nullptr, int nsplit = 0, size_t split_stride = 0) {
-  const size_t off = (size_t)blockIdx.x * kPW + threadIdx.x * 8;
+__device__ __forceinline__ void rmsnorm_row(int row, const u16* x, const u16* y, const float* w, u16* h_out, u16* n_out, float eps,
+                                            const float* ys, int nsplit, size_t split_stride) {
+  const size_t off = (size_t)row * kPW + threadIdx.x * 8;
   __shared__ float s_part[4];
   // every load is issued before the first use: the norm weight, the row and every split's
   // partial (a loop that waited for each split in turn paid one memory round trip per split)
@@ -141,6 +141,19 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const u16* x, const u16* y
   }
   if ((y || ys) && h_out) *reinterpret_cast<u16x8*>(h_out + off) = hv;
   *reinterpret_cast<u16x8*>(n_out + off) = nv;
+}
+
+__global__ __launch_bounds__(256) void rmsnorm_kernel(const u16* x, const u16* y, const float* w, u16* h_out, u16* n_out, float eps,
+                                                      const float* ys = nullptr, int nsplit = 0, size_t split_stride = 0) {
+  rmsnorm_row(blockIdx.x, x, y, w, h_out, n_out, eps, ys, nsplit, split_stride);
+}
+
+// The prefill's first launch: a workgroup per sample for its positions and key-valid bytes (a chain of scans,
+// 3.3 us as a launch of its own), the others each one row of the embeddings' RMSNorm.
+__global__ __launch_bounds__(256) void begin_kernel(const uint8_t* pad, int B, int P, int s_pad, int* pos, uint8_t* valid, const u16* x,
+                                                    const float* w, u16* n_out, float eps) {
+  if ((int)blockIdx.x < B) positions(blockIdx.x, pad, P, s_pad, pos, valid);
+  else rmsnorm_row((int)blockIdx.x - B, x, nullptr, w, nullptr, n_out, eps, nullptr, 0, 0);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -802,8 +815,7 @@ int pi05_prefix_forward(pi05_prefix_ctx* c, const void* embeds, const uint8_t* p
   hipStream_t st = static_cast<hipStream_t>(stream);
   const u16* emb = static_cast<const u16*>(embeds);
   const float eps = c->d.rms_eps;
-  positions_kernel<<<p.B, 256, 0, st>>>(prefix_pad, p.P, p.s_pad, c->pos, c->valid);
-  rmsnorm_kernel<<<p.M, 256, 0, st>>>(emb, nullptr, c->ln, nullptr, c->n, eps);
+  begin_kernel<<<p.B + p.M, 256, 0, st>>>(prefix_pad, p.B, p.P, p.s_pad, c->pos, c->valid, emb, c->ln, c->n, eps);
   // c->h = x + A . W^T, c->n = RMSNorm(c->h) with weight nw (NULL: the last layer's, which nothing reads)
   auto residual = [&](bool lib, const GemmPlan& g, const MmPlan& m, const u16* W, const u16* A, int K, const u16* x, const float* nw) {
     const bool parts = !lib && m.split > 1;
