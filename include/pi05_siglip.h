@@ -5,9 +5,10 @@
  * embeddings the prefill (pi05_prefill.h) consumes.
  *
  * One context (`pi05_vision_ctx`) owns the packed tower weights, the activations of one image
- * count and its GEMM plans.  The plain GEMMs (patch embedding in fp32, q|k|v, out_proj, fc1, fc2,
- * projector with their biases) run on hipBLASLt; LayerNorm, the attention (16 heads of 72) and
- * GELU are hand-written gfx950 kernels.  Conventions are those of pi05_denoise.h.
+ * count and its product plans.  The patch embedding, the products with their biases, LayerNorm, the
+ * attention (16 heads of 72) and GELU are hand-written gfx950 kernels; above 1024 rows q|k|v, out_proj,
+ * fc2 and the projector run on hipBLASLt where it measured faster at creation.  Conventions are those
+ * of pi05_denoise.h.
  */
 #ifndef PI05_SIGLIP_H
 #define PI05_SIGLIP_H

@@ -3,8 +3,8 @@ benchmark driver ``denoise_bench``.
 
 * ``libpi05_denoise.so``: the denoise engine (include/pi05_denoise.h), hand-written kernels only;
 * ``libpi05_prefix.so``: the prefix prefill and the vision tower (include/pi05_prefill.h,
-  include/pi05_siglip.h), whose plain GEMMs run on hipBLASLt -- the only library that links it, so
-  a denoise-only process never loads hipBLASLt.
+  include/pi05_siglip.h), some of whose larger products run on hipBLASLt -- the only library that links
+  it, so a denoise-only process never loads hipBLASLt.
 
     python pi05-infer_amd/build_lib.py [--verbose]
     python pi05-infer_amd/build_lib.py --stamps   (the profiling build phase_stamps.py reads)

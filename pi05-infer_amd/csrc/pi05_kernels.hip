@@ -42,8 +42,8 @@ __global__ void pack_weight_kernel(const u16* __restrict__ src, u16* __restrict_
 // cache keys [0, P); the keys behind them are zeroed so padded lanes never carry NaN/Inf into the masked MFMA
 // products (the graph schedule's action-token keys among them, which every step's qkv projection writes
 // before its attention reads them).  Bound by memory: a V fragment's 16 bytes hold 8 keys of one dim, so
-// the block goes through LDS and every store is 16 bytes (2-byte stores straight from the rows took 22.5 us at
-// 18 layers of 968 keys, this 9).
+// the block goes through LDS and every store is 16 bytes (at 18 layers of 968 keys 2-byte stores straight from the
+// rows took 22.5 us and the tables another 20.8; the one launch takes 10.2).
 //
 // Table workgroups, kTabWgs per sample, kTabToks tokens each: positions sum(pad) + t (engine.py:476-477), key-valid
 // mask, bf16 RoPE tables.  Bound by the sines and cosines (one workgroup per sample took 19 us); each
