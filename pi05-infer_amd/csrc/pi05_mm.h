@@ -52,6 +52,7 @@ struct MmArgs {
   int M, N, K;
   int lda, ldw, ldc;  // row lengths in elements (split s of kMmF32 at C + s M ldc)
   int split;          // K splits (kMmF32), each a run of whole k-tiles
+  int cold;           // 1: W comes from HBM (mm_cold)
 };
 
 typedef __amdgpu_buffer_rsrc_t mm_rsrc;
@@ -455,6 +456,23 @@ __global__ __launch_bounds__(512 + NP * 64) void mm_pw_kernel(MmArgs a) {
 #pragma unroll
     for (int m = 0; m < FM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   MmFrags<FM, FN> f;
+  // Where W comes from HBM: its k-tiles behind the ring's first ones into this XCD's L2, one 128-byte line a
+  // load, shared with the band's other m-tiles.  The multiplying waves have nothing to do yet, and every copy after the
+  // first few finds its line near instead of waiting for HBM with only the ring in flight (27 layers of M = 768: 12 %
+  // of the tower).  Weights that stay in the 256 MB cache behind the L2s gain nothing and pay for the loads (6 layers: 2 %).
+  // The values are not used.
+  constexpr int kPf = 4;
+  uint32_t pf[kPf];
+  {
+    const int tm = (a.M + BM - 1) / BM, share = tm < kMmBand ? tm : kMmBand, lines = BN * (T - (S - 1));
+    const u16* wp = a.W + (size_t)n0 * a.ldw + (size_t)(t0 + S - 1) * 64;
+#pragma unroll
+    for (int j = 0; j < kPf; ++j) {
+      const int i = m_t % share + share * (tid + j * 512), kt = i / BN, row = i % BN < a.N - 1 - n0 ? i % BN : a.N - 1 - n0;
+      pf[j] = 0;
+      if (a.cold && i < lines) pf[j] = *reinterpret_cast<const uint32_t*>(wp + (size_t)row * a.ldw + kt * 64);
+    }
+  }
   mm_barrier();
   int st = grp;
   if (grp) mm_barrier();
@@ -474,6 +492,8 @@ __global__ __launch_bounds__(512 + NP * 64) void mm_pw_kernel(MmArgs a) {
     st = st + 2 >= S ? st + 2 - S : st + 2;
   }
   if ((T & 1) == grp) mm_barrier();  // T + 1 slots for either group
+#pragma unroll
+  for (int j = 0; j < kPf; ++j) asm volatile("" ::"v"(pf[j]));
   // group 0 finishes the m-tiles below FM / 2 of each wave tile, group 1 the others: sum = group 0's + group 1's
   constexpr int HM = FM / 2;
   float* red = reinterpret_cast<float*>(lds) + (size_t)wq * (FM * FN * 256) + lane * 4;
@@ -565,6 +585,9 @@ inline bool mm_launch(int cfg, int epi, const MmArgs& a, hipStream_t st) {
     default: return false;
   }
 }
+
+// Whether layers' weights of this many bytes in all come from HBM on every pass: more than the memory-side cache keeps.
+inline int mm_cold(size_t weight_bytes) { return weight_bytes > (256ull << 20) ? 1 : 0; }
 
 // Holds the stream for `ticks` of the 100 MHz counter (or the bounded number of polls).
 static __global__ void mm_hold_kernel(unsigned ticks) {

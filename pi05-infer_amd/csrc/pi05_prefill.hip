@@ -428,7 +428,7 @@ struct LayerBind {
 
 // Device layout of one context: sizes in bytes.
 struct PrefixPlan {
-  int L = 0, B = 0, P = 0, M = 0, s_pad = 0, n_mt = 0, items = 0, nsplit = 1;
+  int L = 0, B = 0, P = 0, M = 0, s_pad = 0, n_mt = 0, items = 0, nsplit = 1, cold = 0;
   size_t w, ln, h, n, y, qkv, attn, act, qf, kv, pos, valid, invf, rtab, ws, po, pml, dpart;
   size_t total() const {
     return w + ln + 3 * h + qkv + attn + act + qf + 2 * kv + pos + valid + invf + rtab + ws + po + pml + dpart + 16 * 256;
@@ -453,6 +453,7 @@ PrefixPlan plan_of(const pi05_prefix_dims& d) {
   if (p.nsplit < 1) p.nsplit = 1;
   const size_t M = p.M;
   p.w = rup((size_t)p.L * kPLayerElems * 2);
+  p.cold = mm_cold(p.w);
   p.ln = rup((size_t)p.L * 2 * kPW * 4);
   p.h = rup(M * kPW * 2);
   p.qkv = rup(M * kPQkvN * 2);
@@ -553,7 +554,7 @@ int gemm(pi05_prefix_ctx* c, const GemmPlan& p, const u16* W, const u16* A, void
 
 // One product of the layer loop: C[M, N] = A[M, K] . W[N, K]^T with epilogue epi.
 int mm(pi05_prefix_ctx* c, const MmPlan& p, int epi, const u16* W, const u16* A, void* C, int N, int K, int ldc, hipStream_t st) {
-  if (!mm_launch(p.cfg, epi, {A, W, C, nullptr, c->plan.M, N, K, K, K, ldc, p.split}, st)) return fail(c, PI05_E_HIP, "product launch failed");
+  if (!mm_launch(p.cfg, epi, {A, W, C, nullptr, c->plan.M, N, K, K, K, ldc, p.split, c->plan.cold}, st)) return fail(c, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
 
@@ -677,15 +678,15 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
   const float part_ms = (float)(4.0 * M * kPW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kPW / 4e12 * 1e3);
   auto tune_n = [&](const u16* A, int K, MmPlan* o) {  // o_proj, down_proj: one product, or fp32 K splits
     MmPlan one, sp;
-    if (!mm_tune({A, c->w, c->y, nullptr, M, kPW, K, K, K, kPW, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &one) ||
-        !mm_tune({A, c->w, c->dpart, nullptr, M, kPW, K, K, K, kPW, 1}, kMmF32, 2, max_splits(M), part_ms, ls, nl, nullptr, &sp))
+    if (!mm_tune({A, c->w, c->y, nullptr, M, kPW, K, K, K, kPW, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &one) ||
+        !mm_tune({A, c->w, c->dpart, nullptr, M, kPW, K, K, K, kPW, 1, p.cold}, kMmF32, 2, max_splits(M), part_ms, ls, nl, nullptr, &sp))
       return false;
     *o = sp.ms + part_ms * (float)sp.split - bf_ms < one.ms ? sp : one;
     return true;
   };
-  bool tuned = mm_tune({c->n, c->w, c->qkv, nullptr, M, kPQkvN, kPW, kPW, kPW, kPQkvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
-               mm_tune({c->n, c->w, c->qkv, nullptr, M, kPKvN, kPW, kPW, kPW, kPKvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_kv) &&
-               mm_tune({c->n, c->w, c->act, nullptr, M, kPGuN, kPW, kPW, kPW, kPI, 1}, kMmGeglu, 1, 1, 0.f, ls, nl, nullptr, &c->m_gu) &&
+  bool tuned = mm_tune({c->n, c->w, c->qkv, nullptr, M, kPQkvN, kPW, kPW, kPW, kPQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+               mm_tune({c->n, c->w, c->qkv, nullptr, M, kPKvN, kPW, kPW, kPW, kPKvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_kv) &&
+               mm_tune({c->n, c->w, c->act, nullptr, M, kPGuN, kPW, kPW, kPW, kPI, 1, p.cold}, kMmGeglu, 1, 1, 0.f, ls, nl, nullptr, &c->m_gu) &&
                tune_n(c->attn, kPHD, &c->m_o) && tune_n(c->act, kPI, &c->m_d);
   if (tuned && lib) {
     tuned = tune_plan(c->lt, &c->g_qkv, c->w, c->n, c->qkv, c->ws, nullptr, nullptr, ls, nl) &&
@@ -852,7 +853,7 @@ int pi05_prefix_forward(pi05_prefix_ctx* c, const void* embeds, const uint8_t* p
 
 int pi05_debug_product(int cfg, int epi, const void* a, const void* w, void* c, const float* bias, int M, int N, int K, int lda, int ldw,
                        int ldc, int split, void* stream) {
-  const MmArgs args{static_cast<const u16*>(a), static_cast<const u16*>(w), c, bias, M, N, K, lda, ldw, ldc, split};
+  const MmArgs args{static_cast<const u16*>(a), static_cast<const u16*>(w), c, bias, M, N, K, lda, ldw, ldc, split, 1};
   if (!a || !w || !c || epi < kMmBf16 || epi > kMmGeglu || !mm_fits(cfg, epi, args)) return fail(nullptr, PI05_E_INVALID, "the tile does not take this product");
   if (!mm_launch(cfg, epi, args, static_cast<hipStream_t>(stream))) return fail(nullptr, PI05_E_HIP, "product launch failed");
   return PI05_OK;

@@ -340,7 +340,7 @@ struct VLayerBind {
 };
 
 struct VisionPlan {
-  int L = 0, N = 0, M = 0;
+  int L = 0, N = 0, M = 0, cold = 0;
   size_t w, par, head, h, qkv, act, part, ws;
   size_t total() const { return w + par + head + 4 * h + qkv + act + part + ws + 16 * 256; }
 };
@@ -352,6 +352,7 @@ VisionPlan vplan_of(const pi05_vision_dims& d) {
   p.L = d.depth, p.N = d.n_images, p.M = d.n_images * kVS;
   const size_t M = p.M;
   p.w = vrup((size_t)p.L * kVLayerElems * 2);
+  p.cold = mm_cold(p.w);
   p.par = vrup((size_t)p.L * kVLayerParams * 4);
   // heads: packed patch_w + patch_b + pos [256, W] + post w/b (fp32), proj_w bf16, proj_b fp32
   p.head = vrup(((size_t)kVW * kVSteps * 16 + kVW + (size_t)kVS * kVW + 2 * kVW + kVProj) * 4 + (size_t)kVProj * kVW * 2);
@@ -430,6 +431,7 @@ int vgemm(pi05_vision_ctx* c, const GemmPlan& p, const void* W, const void* A, v
 
 int vmm(pi05_vision_ctx* c, const MmPlan& p, int epi, MmArgs a, hipStream_t st) {
   a.split = p.split;
+  a.cold = c->plan.cold;
   if (!mm_launch(p.cfg, epi, a, st)) return vfail(c, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
@@ -528,14 +530,14 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
     // what a reader of fp32 partials pays per split: 4 bytes per output element at ~4 TB/s, less the
     // bf16 output it would read and the product write otherwise
     const float part_ms = (float)(4.0 * M * kVW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kVW / 4e12 * 1e3);
-    ok = mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
-         mm_tune({c->n, c->w, c->act, bz, M, kVI, kVW, kVW, kVW, kVIp, 1}, kMmGelu, 1, 1, 0.f, ls, nl, nullptr, &c->m_fc1) &&
+    ok = mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+         mm_tune({c->n, c->w, c->act, bz, M, kVI, kVW, kVW, kVW, kVIp, 1, p.cold}, kMmGelu, 1, 1, 0.f, ls, nl, nullptr, &c->m_fc1) &&
          mm_tune({c->n, c->proj_w, c->act, bz, M, kVProj, kVW, kVW, kVW, kVProj, 1}, kMmBf16, 1, 1, 0.f, 0, 1, nullptr, &c->m_proj);
     // out_proj and fc2: one product with its bias, or fp32 K splits that the LayerNorm adds
     auto tune_n = [&](const u16* A, int K, MmPlan* out) {
       MmPlan one, sp;
-      if (!mm_tune({A, c->w, c->y, bz, M, kVW, K, K, K, kVW, 1}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &one) ||
-          !mm_tune({A, c->w, c->part, nullptr, M, kVW, K, K, K, kVW, 1}, kMmF32, 2, kVMaxSplits, part_ms, ls, nl, nullptr, &sp))
+      if (!mm_tune({A, c->w, c->y, bz, M, kVW, K, K, K, kVW, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &one) ||
+          !mm_tune({A, c->w, c->part, nullptr, M, kVW, K, K, K, kVW, 1, p.cold}, kMmF32, 2, kVMaxSplits, part_ms, ls, nl, nullptr, &sp))
         return false;
       *out = sp.ms + part_ms * (float)sp.split - bf_ms < one.ms ? sp : one;
       return true;
