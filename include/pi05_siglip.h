@@ -68,6 +68,12 @@ int pi05_vision_refresh_weights(pi05_vision_ctx* ctx, void* stream);
  * Enqueues only. */
 int pi05_vision_forward(pi05_vision_ctx* ctx, const float* pixels, void* out, void* stream);
 
+/* What the context chose for a product when it was created (a debug hook).  which: 0 q|k|v, 1 out_proj,
+ * 2 fc1, 3 fc2, 4 projector.  choice[4]: the tile (pi05_debug_product's cfg), its K splits, 1 if it was timed and
+ * runs with weights that come from HBM, 1 if hipBLASLt runs the product instead.  us[2]: the tile's time alone,
+ * and hipBLASLt's (0 where it was no candidate). */
+int pi05_vision_product(pi05_vision_ctx* ctx, int which, int32_t* choice, float* us);
+
 #ifdef __cplusplus
 }
 #endif

@@ -597,9 +597,10 @@ static __global__ void mm_hold_kernel(unsigned ticks) {
 #endif
 }
 
-// The tile and the K split of one product.
+// The tile and the K split of one product, and whether W comes from HBM (MmArgs::cold): a product is launched as
+// it was timed.
 struct MmPlan {
-  int cfg = -1, split = 1;
+  int cfg = -1, split = 1, cold = 0;
   float ms = 1e30f;  // time of the product alone
 };
 
@@ -643,7 +644,7 @@ inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_
   for (int cfg = 0; cfg < kMmCfgs && ok; ++cfg)
     for (int s = smin; s <= smax && ok; ++s) {
       MmPlan p;
-      p.cfg = cfg, p.split = a.split = s;
+      p.cfg = cfg, p.split = a.split = s, p.cold = a.cold;
       a.W = w;
       if (!mm_fits(cfg, epi, a) || (s > 1 && a.K / 64 / s < 4)) continue;
       ok = time(p, 6, &p.ms);

@@ -554,7 +554,7 @@ int gemm(pi05_prefix_ctx* c, const GemmPlan& p, const u16* W, const u16* A, void
 
 // One product of the layer loop: C[M, N] = A[M, K] . W[N, K]^T with epilogue epi.
 int mm(pi05_prefix_ctx* c, const MmPlan& p, int epi, const u16* W, const u16* A, void* C, int N, int K, int ldc, hipStream_t st) {
-  if (!mm_launch(p.cfg, epi, {A, W, C, nullptr, c->plan.M, N, K, K, K, ldc, p.split, c->plan.cold}, st)) return fail(c, PI05_E_HIP, "product launch failed");
+  if (!mm_launch(p.cfg, epi, {A, W, C, nullptr, c->plan.M, N, K, K, K, ldc, p.split, p.cold}, st)) return fail(c, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
 

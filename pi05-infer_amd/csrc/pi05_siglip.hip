@@ -431,7 +431,7 @@ int vgemm(pi05_vision_ctx* c, const GemmPlan& p, const void* W, const void* A, v
 
 int vmm(pi05_vision_ctx* c, const MmPlan& p, int epi, MmArgs a, hipStream_t st) {
   a.split = p.split;
-  a.cold = c->plan.cold;
+  a.cold = p.cold;
   if (!mm_launch(p.cfg, epi, a, st)) return vfail(c, PI05_E_HIP, "product launch failed");
   return PI05_OK;
 }
@@ -524,7 +524,9 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
                      make_plan(c->lt, M, kVProj, kVW, kVWorkspace, &c->g_proj, &perr, bias));
   if (ok) {
     const float* bz = c->par;  // any fp32 vector long enough (zeros) stands in for the biases while timing
-    // (weights rotate over the layers' blocks while timing, as the layer loop streams them)
+    // (weights rotate over the layers' blocks while timing, as the layer loop streams them; the projector's too:
+    // the tower's weights have passed through the caches since its own were read)
+    static_assert((size_t)kVProj * kVW <= kVLayerElems, "the projector is timed on the layers' blocks");
     const size_t ls = kVLayerElems * 2;
     const int nl = p.L;
     // what a reader of fp32 partials pays per split: 4 bytes per output element at ~4 TB/s, less the
@@ -532,7 +534,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
     const float part_ms = (float)(4.0 * M * kVW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kVW / 4e12 * 1e3);
     ok = mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
          mm_tune({c->n, c->w, c->act, bz, M, kVI, kVW, kVW, kVW, kVIp, 1, p.cold}, kMmGelu, 1, 1, 0.f, ls, nl, nullptr, &c->m_fc1) &&
-         mm_tune({c->n, c->proj_w, c->act, bz, M, kVProj, kVW, kVW, kVW, kVProj, 1}, kMmBf16, 1, 1, 0.f, 0, 1, nullptr, &c->m_proj);
+         mm_tune({c->n, c->w, c->act, bz, M, kVProj, kVW, kVW, kVW, kVProj, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_proj);
     // out_proj and fc2: one product with its bias, or fp32 K splits that the LayerNorm adds
     auto tune_n = [&](const u16* A, int K, MmPlan* out) {
       MmPlan one, sp;
@@ -547,7 +549,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
       ok = tune_plan(c->lt, &c->g_qkv, c->w, c->n, c->qkv, c->ws, nullptr, bz, ls, nl) &&
            tune_plan(c->lt, &c->g_o, c->w, c->attn, c->y, c->ws, nullptr, bz, ls, nl) &&
            tune_plan(c->lt, &c->g_fc2, c->w, c->act, c->y, c->ws, nullptr, bz, ls, nl) &&
-           tune_plan(c->lt, &c->g_proj, c->proj_w, c->n, c->act, c->ws, nullptr, bz);
+           tune_plan(c->lt, &c->g_proj, c->w, c->n, c->act, c->ws, nullptr, bz, ls, nl);
       auto cost = [&](const MmPlan& m) { return m.split > 1 ? m.ms + part_ms * (float)m.split - bf_ms : m.ms; };
       c->lib_qkv = c->g_qkv.ms < c->m_qkv.ms;
       c->lib_o = c->g_o.ms < cost(c->m_o);
@@ -562,6 +564,17 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
     return vfail(nullptr, PI05_E_HIP, perr);
   }
   *out = c;
+  return PI05_OK;
+}
+
+int pi05_vision_product(pi05_vision_ctx* c, int which, int32_t* choice, float* us) {
+  if (!c) return vfail(nullptr, PI05_E_INVALID, "ctx is NULL");
+  if (which < 0 || which > 4 || !choice || !us) return vfail(c, PI05_E_INVALID, "which must be in [0, 4], choice and us non-NULL");
+  const MmPlan* const m[5] = {&c->m_qkv, &c->m_o, &c->m_fc1, &c->m_fc2, &c->m_proj};
+  const GemmPlan* const g[5] = {&c->g_qkv, &c->g_o, nullptr, &c->g_fc2, &c->g_proj};
+  const bool lib[5] = {c->lib_qkv, c->lib_o, false, c->lib_fc2, c->lib_proj};
+  choice[0] = m[which]->cfg, choice[1] = m[which]->split, choice[2] = m[which]->cold, choice[3] = lib[which];
+  us[0] = m[which]->ms * 1e3f, us[1] = g[which] ? g[which]->ms * 1e3f : 0.f;
   return PI05_OK;
 }
 

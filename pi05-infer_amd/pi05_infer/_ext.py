@@ -83,6 +83,7 @@ VISION_EXPORTED_SYMBOLS = (
     "pi05_vision_bind_heads",
     "pi05_vision_refresh_weights",
     "pi05_vision_forward",
+    "pi05_vision_product",
 )
 
 
@@ -239,6 +240,7 @@ def load_prefix_library(path: str = PREFIX_LIB_PATH) -> ctypes.CDLL:
         "pi05_vision_bind_heads": (i32, [vp] + [vp] * 7),
         "pi05_vision_refresh_weights": (i32, [vp, vp]),
         "pi05_vision_forward": (i32, [vp, vp, vp, vp]),
+        "pi05_vision_product": (i32, [vp, i32, ctypes.POINTER(i32), ctypes.POINTER(ctypes.c_float)]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(lib, name)
@@ -633,6 +635,16 @@ def vision_device_bytes(dims: Pi05VisionDims) -> int:
     return int(load_prefix_library().pi05_vision_device_bytes(ctypes.byref(dims)))
 
 
+def _product_choices(fn, check, handle, names) -> dict:
+    """Per product what its context chose at creation: tile, splits, cold, library, us, library_us."""
+    choice, us = (ctypes.c_int32 * 4)(), (ctypes.c_float * 2)()
+    out = {}
+    for i, name in enumerate(names):
+        check(fn(handle, i, choice, us))
+        out[name] = dict(tile=choice[0], splits=choice[1], cold=bool(choice[2]), library=bool(choice[3]), us=us[0], library_us=us[1])
+    return out
+
+
 class VisionContext:
     """One SigLIP + projector context: an image count on the current device."""
 
@@ -684,6 +696,9 @@ class VisionContext:
         op = _ptr(out, torch.bfloat16, "out", self.device)
         self._call(self.lib.pi05_vision_forward(self.handle, pp, op, _stream_ptr(stream)))
         return out
+
+    def products(self) -> dict:
+        return _product_choices(self.lib.pi05_vision_product, self._call, self.handle, ("qkv", "out_proj", "fc1", "fc2", "projector"))
 
     def close(self) -> None:
         if getattr(self, "handle", None):
