@@ -104,6 +104,10 @@ int pi05_prefix_forward(pi05_prefix_ctx* ctx, const void* embeds, const uint8_t*
                         void* const* k_layers, void* const* v_layers, int64_t kv_batch_stride,
                         int64_t kv_row_stride, void* stream);
 
+/* What the context chose for a product when it was created (a debug hook).  which: 0 q|k|v, 1 k|v (the last
+ * layer's), 2 o_proj, 3 gate|up, 4 down_proj; choice and us as for pi05_vision_product (pi05_siglip.h). */
+int pi05_prefix_product(pi05_prefix_ctx* ctx, int which, int32_t* choice, float* us);
+
 /* One matrix product of the prefill and the vision tower on its own (a parity / debug hook):
  * C[M, N] = A[M, K] . W[N, K]^T, bf16 operands with rows of lda / ldw elements, on tile `cfg`
  * (0 .. 7) with epilogue `epi` (0: bf16, optional fp32 bias[N]; 1: the same through GELU; 2: fp32

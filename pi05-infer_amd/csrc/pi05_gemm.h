@@ -110,8 +110,8 @@ inline hipblasStatus_t run_plan(hipblasLtHandle_t h, const GemmPlan& p, const hi
   return hipblasLtMatmul(h, p.desc, &alpha, W, p.lw, A, p.la, &beta, C, p.lc, C, p.lc, &algo, ws, ws_bytes, st);
 }
 
-// Time every candidate algorithm on real buffers (2 runs after one warm-up; values do not affect
-// the timing), re-time the 6 fastest and keep the best; candidates that fail to launch are skipped.  w_stride / w_count: see w_at below.
+// Time every candidate algorithm on the caller's buffers (2 runs after one warm-up; random values, on which a
+// large product's clock is the one of real operands), re-time the 6 fastest and keep the best; candidates that fail to launch are skipped.  w_stride / w_count: see w_at below.
 inline bool tune_plan(hipblasLtHandle_t h, GemmPlan* p, const void* W, const void* A, void* C, void* ws, hipStream_t st,
                       const float* bias = nullptr, size_t w_stride = 0, int w_count = 1) {
   // run r reads the weights at W + (r mod w_count) * w_stride: with one weight block per layer the

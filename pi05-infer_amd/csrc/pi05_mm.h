@@ -604,10 +604,28 @@ struct MmPlan {
   float ms = 1e30f;  // time of the product alone
 };
 
+// Operands for timing: normal values, as activations and weights are.  Zeros will not do: they switch little in the
+// matrix cores, so a large tile keeps a clock that it does not have in use (gate|up and its GeGLU, M = 1024: 88 us
+// on zeros, 102 on values of four exponents, 113 on normal ones; tiles up to 128 x 128: the same).  On zeros
+// down_proj at 968 rows took 192 x 256 (62 us on random values) in place of 256 x 192 (59).
+static __global__ __launch_bounds__(256) void mm_random_kernel(u16* p, size_t n, float std) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    uint64_t h = (i + 1) * 0x9e3779b97f4a7c15ull;
+    h = (h ^ (h >> 32)) * 0xd6e8feb86659fd93ull;
+    h ^= h >> 32;
+    const float u = ((float)(h & 0xffffff) + 0.5f) * 0x1p-24f, v = (float)((h >> 24) & 0xffffff) * 0x1p-24f;
+    p[i] = f2bf(std * sqrtf(-2.0f * __logf(u)) * __cosf(6.2831853f * v));
+  }
+}
+inline bool mm_random(u16* p, size_t n, float std, hipStream_t st) {
+  mm_random_kernel<<<4096, 256, 0, st>>>(p, n, std);
+  return hipGetLastError() == hipSuccess;
+}
+
 // The fastest tile and K split for a product: every tile with every split in [smin, smax] that leaves a split
-// at least 4 k-tiles, timed on the caller's buffers as the layer loop runs them (run r reads the weights at
-// a.W + (r mod w_count) * w_stride bytes, so they stream from memory; values do not affect the choice of
-// path), the 6 fastest again in 4 interleaved rounds of 20 runs.  The stream is held while the host
+// at least 4 k-tiles, timed on the caller's buffers (random values: see mm_random_kernel) as the layer loop runs
+// them (run r reads the weights at a.W + (r mod w_count) * w_stride bytes, so from beyond the L2s), the 6 fastest
+// again in 4 interleaved rounds of 20 runs.  The stream is held while the host
 // enqueues the runs: a 6 us product is otherwise timed at the rate the host launches it, where all tiles look
 // alike (the picks of a 256-row layer then changed from context to context).  Timed rather than computed
 // from the sizes because two effects of equal size decide: how evenly the tiles fill 256 CUs (M = 768, N =

@@ -640,21 +640,10 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
   c->po = reinterpret_cast<float*>(take(p.po));
   c->pml = reinterpret_cast<float*>(take(p.pml));
   c->dpart = reinterpret_cast<float*>(take(p.dpart));
-  // everything starts zeroed: query rows and keys past P stay zero (finite and masked) for the
-  // life of the context, and the GEMM tuning below reads defined values
-  e = hipMemset(c->base, 0, p.total());
+  e = hipMemset(c->base, 0, p.total());  // defined values wherever the tuning below reads
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&c->host_bad), sizeof(unsigned), hipHostMallocMapped);
   if (e == hipSuccess) *c->host_bad = 0;
-  float invf[kHalfDim];
-  prefix_inv_freq(dims->rope_theta, invf);
-  if (e == hipSuccess) e = hipMemcpy(c->inv_freq, invf, sizeof(invf), hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    rope_table_kernel<<<p.P + 1, kHalfDim>>>(c->inv_freq, p.P, c->rope_tab);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipDeviceSynchronize();
-  }
   if (e != hipSuccess) {
-    if (c->host_bad) (void)hipHostFree(c->host_bad);
     hipFree(c->base);
     delete c;
     return fail(nullptr, PI05_E_HIP, std::string("prefix context initialisation failed: ") + hipGetErrorString(e));
@@ -684,7 +673,9 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
     *o = sp.ms + part_ms * (float)sp.split - bf_ms < one.ms ? sp : one;
     return true;
   };
-  bool tuned = mm_tune({c->n, c->w, c->qkv, nullptr, M, kPQkvN, kPW, kPW, kPW, kPQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+  bool tuned = mm_random(c->w, (size_t)nl * kPLayerElems, 0.02f, nullptr) && mm_random(c->n, (size_t)M * kPW, 1.f, nullptr) &&
+               mm_random(c->attn, (size_t)M * kPHD, 1.f, nullptr) && mm_random(c->act, (size_t)M * kPI, 1.f, nullptr) &&
+               mm_tune({c->n, c->w, c->qkv, nullptr, M, kPQkvN, kPW, kPW, kPW, kPQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
                mm_tune({c->n, c->w, c->qkv, nullptr, M, kPKvN, kPW, kPW, kPW, kPKvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_kv) &&
                mm_tune({c->n, c->w, c->act, nullptr, M, kPGuN, kPW, kPW, kPW, kPI, 1, p.cold}, kMmGeglu, 1, 1, 0.f, ls, nl, nullptr, &c->m_gu) &&
                tune_n(c->attn, kPHD, &c->m_o) && tune_n(c->act, kPI, &c->m_d);
@@ -703,7 +694,33 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
     pi05_prefix_destroy(c);
     return fail(nullptr, PI05_E_HIP, "GEMM tuning failed");
   }
+  // from here on everything is zero but the tables: query rows and keys past P stay so (finite and masked) for the
+  // life of the context
+  float invf[kHalfDim];
+  prefix_inv_freq(dims->rope_theta, invf);
+  e = hipMemset(c->base, 0, p.total());
+  if (e == hipSuccess) e = hipMemcpy(c->inv_freq, invf, sizeof(invf), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    rope_table_kernel<<<p.P + 1, kHalfDim>>>(c->inv_freq, p.P, c->rope_tab);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+  }
+  if (e != hipSuccess) {
+    pi05_prefix_destroy(c);
+    return fail(nullptr, PI05_E_HIP, std::string("prefix context initialisation failed: ") + hipGetErrorString(e));
+  }
   *out = c;
+  return PI05_OK;
+}
+
+int pi05_prefix_product(pi05_prefix_ctx* c, int which, int32_t* choice, float* us) {
+  if (!c) return fail(nullptr, PI05_E_INVALID, "ctx is NULL");
+  if (which < 0 || which > 4 || !choice || !us) return fail(c, PI05_E_INVALID, "which must be in [0, 4], choice and us non-NULL");
+  const MmPlan* const m[5] = {&c->m_qkv, &c->m_kv, &c->m_o, &c->m_gu, &c->m_d};
+  const GemmPlan* const g[5] = {&c->g_qkv, &c->g_kv, &c->g_o, nullptr, &c->g_d};
+  const bool lib[5] = {c->lib_qkv, c->lib_kv, c->lib_o, false, c->lib_d};
+  choice[0] = m[which]->cfg, choice[1] = m[which]->split, choice[2] = m[which]->cold, choice[3] = lib[which];
+  us[0] = m[which]->ms * 1e3f, us[1] = g[which] ? g[which]->ms * 1e3f : 0.f;
   return PI05_OK;
 }
 

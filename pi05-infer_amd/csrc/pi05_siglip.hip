@@ -505,7 +505,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   c->act = reinterpret_cast<u16*>(take(p.act));
   c->part = reinterpret_cast<float*>(take(p.part));
   c->ws = take(p.ws);
-  // zeroed once: tuning reads defined data
+  // defined values wherever the tuning below reads (zero biases)
   e = hipMemset(c->base, 0, p.total());
   if (e != hipSuccess) {
     hipFree(c->base);
@@ -532,7 +532,9 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
     // what a reader of fp32 partials pays per split: 4 bytes per output element at ~4 TB/s, less the
     // bf16 output it would read and the product write otherwise
     const float part_ms = (float)(4.0 * M * kVW / 4e12 * 1e3), bf_ms = (float)(2.0 * M * kVW / 4e12 * 1e3);
-    ok = mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
+    ok = mm_random(c->w, (size_t)nl * kVLayerElems, 0.02f, nullptr) && mm_random(c->n, M * (size_t)kVW, 1.f, nullptr) &&
+         mm_random(c->attn, M * (size_t)kVW, 1.f, nullptr) && mm_random(c->act, M * (size_t)kVIp, 1.f, nullptr) &&
+         mm_tune({c->n, c->w, c->qkv, bz, M, kVQkvN, kVW, kVW, kVW, kVQkvN, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_qkv) &&
          mm_tune({c->n, c->w, c->act, bz, M, kVI, kVW, kVW, kVW, kVIp, 1, p.cold}, kMmGelu, 1, 1, 0.f, ls, nl, nullptr, &c->m_fc1) &&
          mm_tune({c->n, c->w, c->act, bz, M, kVProj, kVW, kVW, kVW, kVProj, 1, p.cold}, kMmBf16, 1, 1, 0.f, ls, nl, nullptr, &c->m_proj);
     // out_proj and fc2: one product with its bias, or fp32 K splits that the LayerNorm adds
@@ -562,6 +564,13 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
     if (perr.empty()) perr = "hipblasLtCreate failed";
     pi05_vision_destroy(c);
     return vfail(nullptr, PI05_E_HIP, perr);
+  }
+  // the columns past 4304 of fc2's operands are read and never written: zero from here on
+  e = hipMemset(c->base, 0, p.total());
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e != hipSuccess) {
+    pi05_vision_destroy(c);
+    return vfail(nullptr, PI05_E_HIP, std::string("vision context initialisation failed: ") + hipGetErrorString(e));
   }
   *out = c;
   return PI05_OK;

@@ -69,6 +69,7 @@ PREFIX_EXPORTED_SYMBOLS = (
     "pi05_prefix_status",
     "pi05_prefix_forward",
     "pi05_debug_product",
+    "pi05_prefix_product",
 )
 
 # every exported symbol of include/pi05_siglip.h
@@ -240,6 +241,7 @@ def load_prefix_library(path: str = PREFIX_LIB_PATH) -> ctypes.CDLL:
         "pi05_vision_bind_heads": (i32, [vp] + [vp] * 7),
         "pi05_vision_refresh_weights": (i32, [vp, vp]),
         "pi05_vision_forward": (i32, [vp, vp, vp, vp]),
+        "pi05_prefix_product": (i32, [vp, i32, ctypes.POINTER(i32), ctypes.POINTER(ctypes.c_float)]),
         "pi05_vision_product": (i32, [vp, i32, ctypes.POINTER(i32), ctypes.POINTER(ctypes.c_float)]),
     }
     for name, (res, args) in sig.items():
@@ -597,6 +599,9 @@ class PrefixContext:
         self._pad = pad
         self._call(self.lib.pi05_prefix_forward(self.handle, ep, pad.data_ptr(), karr, varr, bstride, rstride,
                                                 _stream_ptr(stream)))
+
+    def products(self) -> dict:
+        return _product_choices(self.lib.pi05_prefix_product, self._call, self.handle, ("qkv", "kv", "o_proj", "gate_up", "down_proj"))
 
     def close(self) -> None:
         if getattr(self, "handle", None):

@@ -20,3 +20,36 @@ def test_projector_is_timed_as_it_runs(depth):
     ctx.close()
     print(got, flush=True)
     assert {n: p["cold"] for n, p in got.items()} == dict.fromkeys(got, depth == 10)
+
+
+def test_tiles_are_timed_on_values_that_switch_the_matrix_cores():
+    """gate|up at 1024 rows (512 tiles of 256 x 256 on 256 CUs) runs faster on zeros than on normal values: the time
+    that the context chose its tile by is that of normal operands.  Measured 0.94 of it here, 0.79 when contexts
+    timed zeros; the line lies between the two."""
+    print("case prefill choices: depth 2, 1 x 1024", flush=True)
+    d = _ext.prefix_default_dims()
+    d.depth, d.batch, d.prefix_len = 2, 1, 1024
+    ctx = _ext.PrefixContext(d, torch.device("cuda"))
+    got = ctx.products()
+    ctx.close()
+    m, n, k = 1024, 32768, 2048
+    a = torch.randn(m, k, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(2, n, k, device="cuda") * 0.02).to(torch.bfloat16)
+    out = torch.empty(m, n // 2, dtype=torch.bfloat16, device="cuda")
+    lib = _ext.load_prefix_library()
+
+    def once(i):
+        assert lib.pi05_debug_product(got["gate_up"]["tile"], 3, a.data_ptr(), w[i % 2].data_ptr(), out.data_ptr(), None, m, n, k, k, k, n // 2, 1,
+                                      torch.cuda.current_stream().cuda_stream) == 0
+
+    best, start, end = 1e9, torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for _ in range(5):
+        once(1)
+        start.record()
+        for i in range(20):
+            once(i)
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) / 20 * 1e3)
+    print(f"chosen by {got['gate_up']['us']:.1f} us, on random operands {best:.1f} us; {got}", flush=True)
+    assert got["gate_up"]["us"] >= 0.87 * best
