@@ -15,6 +15,8 @@
 #include <utility>
 #include <vector>
 
+#include "pi05_mm.h"
+
 namespace pi05 {
 
 struct GemmPlan {
@@ -111,7 +113,8 @@ inline hipblasStatus_t run_plan(hipblasLtHandle_t h, const GemmPlan& p, const hi
 }
 
 // Time every candidate algorithm on the caller's buffers (2 runs after one warm-up; random values, on which a
-// large product's clock is the one of real operands), re-time the 6 fastest and keep the best; candidates that fail to launch are skipped.  w_stride / w_count: see w_at below.
+// large product's clock is the one of real operands), re-time the fastest as mm_tune does, whose result the time is
+// compared with, and keep the best; candidates that fail to launch are skipped.  w_stride / w_count: see w_at below.
 inline bool tune_plan(hipblasLtHandle_t h, GemmPlan* p, const void* W, const void* A, void* C, void* ws, hipStream_t st,
                       const float* bias = nullptr, size_t w_stride = 0, int w_count = 1) {
   // run r reads the weights at W + (r mod w_count) * w_stride: with one weight block per layer the
@@ -124,14 +127,7 @@ inline bool tune_plan(hipblasLtHandle_t h, GemmPlan* p, const void* W, const voi
     return false;
   }
   auto time_algo = [&](const hipblasLtMatmulHeuristicResult_t& c, int reps, float* ms) {
-    bool ok = lt_ok(run_plan(h, *p, c.algo, c.workspaceSize, w_at(w_count - 1), A, C, bias, ws, st));
-    if (!ok) return false;
-    hipEventRecord(e0, st);
-    for (int r = 0; r < reps && ok; ++r) ok = lt_ok(run_plan(h, *p, c.algo, c.workspaceSize, w_at(r), A, C, bias, ws, st));
-    hipEventRecord(e1, st);
-    if (hipEventSynchronize(e1) != hipSuccess || !ok || hipEventElapsedTime(ms, e0, e1) != hipSuccess) return false;
-    *ms /= (float)reps;
-    return true;
+    return mm_time([&](int r) { return lt_ok(run_plan(h, *p, c.algo, c.workspaceSize, w_at(r), A, C, bias, ws, st)); }, reps, e0, e1, st, ms);
   };
   std::vector<std::pair<float, size_t>> timed;
   for (size_t i = 0; i < p->cands.size(); ++i) {
@@ -139,13 +135,13 @@ inline bool tune_plan(hipblasLtHandle_t h, GemmPlan* p, const void* W, const voi
     if (time_algo(p->cands[i], 2, &ms)) timed.emplace_back(ms, i);
   }
   std::sort(timed.begin(), timed.end());
-  // finalists: 3 interleaved rounds of 10 runs each (so clock drift hits them alike), best round kept
-  const size_t nf = timed.size() < 6 ? timed.size() : 6;
+  // finalists: interleaved rounds (so clock drift hits them alike), best round kept
+  const size_t nf = std::min<size_t>(timed.size(), kMmFinalists);
   std::vector<float> score(nf, 1e30f);
-  for (int round = 0; round < 3; ++round)
+  for (int round = 0; round < kMmRounds; ++round)
     for (size_t k = 0; k < nf; ++k) {
       float ms = 0.f;
-      if (time_algo(p->cands[timed[k].second], 10, &ms) && ms < score[k]) score[k] = ms;
+      if (time_algo(p->cands[timed[k].second], kMmRuns, &ms) && ms < score[k]) score[k] = ms;
     }
   float best = 1e30f;
   for (size_t k = 0; k < nf; ++k)

@@ -597,6 +597,22 @@ static __global__ void mm_hold_kernel(unsigned ticks) {
 #endif
 }
 
+// Time of one of `reps` runs in a row (launch(r) enqueues run r), the same for every candidate of a product.  The
+// stream is held while the host enqueues them: a 6 us product is otherwise timed at the rate the host launches it,
+// where all candidates look alike (a 256-row layer's picks then changed from context to context).
+constexpr int kMmFinalists = 6, kMmRounds = 4, kMmRuns = 20;  // the fastest again, in interleaved rounds of so many runs
+template <class F>
+inline bool mm_time(F&& launch, int reps, hipEvent_t e0, hipEvent_t e1, hipStream_t st, float* ms) {
+  if (!launch(reps - 1)) return false;
+  mm_hold_kernel<<<1, 1, 0, st>>>(1500u * (unsigned)reps);  // 15 us a run
+  bool ok = hipEventRecord(e0, st) == hipSuccess;
+  for (int r = 0; r < reps && ok; ++r) ok = launch(r);
+  ok = hipEventRecord(e1, st) == hipSuccess && ok;
+  ok = hipEventSynchronize(e1) == hipSuccess && ok && hipEventElapsedTime(ms, e0, e1) == hipSuccess;
+  *ms /= (float)reps;
+  return ok;
+}
+
 // The tile and the K split of one product, and whether W comes from HBM (MmArgs::cold): a product is launched as
 // it was timed.
 struct MmPlan {
@@ -624,11 +640,8 @@ inline bool mm_random(u16* p, size_t n, float std, hipStream_t st) {
 
 // The fastest tile and K split for a product: every tile with every split in [smin, smax] that leaves a split
 // at least 4 k-tiles, timed on the caller's buffers (random values: see mm_random_kernel) as the layer loop runs
-// them (run r reads the weights at a.W + (r mod w_count) * w_stride bytes, so from beyond the L2s), the 6 fastest
-// again in 4 interleaved rounds of 20 runs.  The stream is held while the host
-// enqueues the runs: a 6 us product is otherwise timed at the rate the host launches it, where all tiles look
-// alike (the picks of a 256-row layer then changed from context to context).  Timed rather than computed
-// from the sizes because two effects of equal size decide: how evenly the tiles fill 256 CUs (M = 768, N =
+// them (run r reads the weights at a.W + (r mod w_count) * w_stride bytes, so from beyond the L2s), the fastest
+// again.  Timed rather than computed from the sizes because two effects of equal size decide: how evenly the tiles fill 256 CUs (M = 768, N =
 // 4304: 128 x 128 12.6 us, 128 x 96 19.6 us) and the copies per MFMA (M = 968, N = 32768: 256 x 256 115 us,
 // 128 x 128 166 us).  split_ms: what the reader of the partial sums pays per split.
 inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_t w_stride, int w_count, hipStream_t st, MmPlan* out) {
@@ -641,17 +654,11 @@ inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_
   const u16* w = a.W;
   auto time = [&](const MmPlan& c, int reps, float* ms) {
     a.split = c.split;
-    a.W = w;
-    bool ok = mm_launch(c.cfg, epi, a, st);
-    mm_hold_kernel<<<1, 1, 0, st>>>(1500u * (unsigned)reps);  // 15 us a run
-    ok = ok && hipEventRecord(e0, st) == hipSuccess;
-    for (int r = 0; r < reps && ok; ++r) {
+    auto launch = [&](int r) {
       a.W = w + (size_t)(r % w_count) * (w_stride / 2);
-      ok = mm_launch(c.cfg, epi, a, st);
-    }
-    ok = ok && hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(ms, e0, e1) == hipSuccess;
-    *ms /= (float)reps;
-    return ok;
+      return mm_launch(c.cfg, epi, a, st);
+    };
+    return mm_time(launch, reps, e0, e1, st, ms);
   };
   std::vector<std::pair<float, MmPlan>> c;
   bool ok = true;
@@ -669,12 +676,12 @@ inline bool mm_tune(MmArgs a, int epi, int smin, int smax, float split_ms, size_
       c.emplace_back(p.ms + split_ms * (float)s, p);
     }
   std::sort(c.begin(), c.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-  const size_t n = c.size() < 6 ? c.size() : 6;
+  const size_t n = std::min<size_t>(c.size(), kMmFinalists);
   for (size_t i = 0; i < n; ++i) c[i].second.ms = 1e30f;
-  for (int round = 0; round < 4 && ok; ++round)
+  for (int round = 0; round < kMmRounds && ok; ++round)
     for (size_t i = 0; i < n && ok; ++i) {
       float ms = 0.f;
-      ok = time(c[i].second, 20, &ms);
+      ok = time(c[i].second, kMmRuns, &ms);
       c[i].second.ms = std::min(c[i].second.ms, ms);
     }
   (void)hipEventDestroy(e0);
