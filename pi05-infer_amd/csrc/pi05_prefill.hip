@@ -434,7 +434,7 @@ struct PrefixPlan {
     return w + ln + 3 * h + qkv + attn + act + qf + 2 * kv + pos + valid + invf + rtab + ws + po + pml + dpart + 16 * 256;
   }
 };
-constexpr size_t kWorkspace = 64ull << 20;
+constexpr size_t kWorkspace = 64ull << 20;  // hipBLASLt's, where it is a candidate
 
 size_t rup(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -465,7 +465,7 @@ PrefixPlan plan_of(const pi05_prefix_dims& d) {
   p.valid = rup((size_t)p.B * p.s_pad);
   p.invf = rup(kHalfDim * 4);
   p.rtab = rup((size_t)(p.P + 1) * kHeadDim * 2);
-  p.ws = kWorkspace;
+  p.ws = p.M > kLibRows ? kWorkspace : 0;
   const size_t rows = (size_t)p.B * p.n_mt * 16;
   p.po = p.nsplit > 1 ? rup((size_t)p.nsplit * rows * kHeadDim * 4) : 0;
   p.pml = p.nsplit > 1 ? rup((size_t)p.nsplit * rows * 2 * 4) : 0;
@@ -636,7 +636,7 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
   c->valid = reinterpret_cast<uint8_t*>(take(p.valid));
   c->inv_freq = reinterpret_cast<float*>(take(p.invf));
   c->rope_tab = reinterpret_cast<u16*>(take(p.rtab));
-  c->ws = take(p.ws);
+  c->ws = p.ws ? take(p.ws) : nullptr;
   c->po = reinterpret_cast<float*>(take(p.po));
   c->pml = reinterpret_cast<float*>(take(p.pml));
   c->dpart = reinterpret_cast<float*>(take(p.dpart));
@@ -650,7 +650,7 @@ int pi05_prefix_create(const pi05_prefix_dims* dims, pi05_prefix_ctx** out) {
   }
   std::string perr;
   const int M = p.M;
-  const bool lib = M > kLibRows;
+  const bool lib = p.ws != 0;
   if (lib && (!lt_ok(hipblasLtCreate(&c->lt)) || !make_plan(c->lt, M, kPQkvN, kPW, kWorkspace, &c->g_qkv, &perr) ||
               !make_plan(c->lt, M, kPKvN, kPW, kWorkspace, &c->g_kv, &perr) || !make_plan(c->lt, M, kPW, kPHD, kWorkspace, &c->g_o, &perr) ||
               !make_plan(c->lt, M, kPW, kPI, kWorkspace, &c->g_d, &perr))) {

@@ -42,7 +42,7 @@ constexpr size_t kVOffQkv = 0, kVOffO = kVOffQkv + (size_t)kVQkvN * kVW, kVOff1 
 constexpr size_t kVPOffBqkv = 0, kVPOffBo = kVQkvN, kVPOffB1 = kVPOffBo + kVW, kVPOffB2 = kVPOffB1 + kVI,
                  kVPOffLn1w = kVPOffB2 + kVW, kVPOffLn1b = kVPOffLn1w + kVW, kVPOffLn2w = kVPOffLn1b + kVW,
                  kVPOffLn2b = kVPOffLn2w + kVW, kVLayerParams = kVPOffLn2b + kVW;
-constexpr size_t kVWorkspace = 32ull << 20;
+constexpr size_t kVWorkspace = 32ull << 20;  // hipBLASLt's, where it is a candidate
 constexpr int kVMaxSplits = 8;  // K splits of out_proj and fc2 at most
 // rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate
 constexpr int kVLibRows = 1024;
@@ -360,7 +360,7 @@ VisionPlan vplan_of(const pi05_vision_dims& d) {
   p.qkv = vrup(M * kVQkvN * 2);
   p.part = vrup((size_t)kVMaxSplits * M * kVW * 4);
   p.act = vrup(M * kVIp * 2);
-  p.ws = kVWorkspace;
+  p.ws = p.M > kVLibRows ? kVWorkspace : 0;
   return p;
 }
 
@@ -504,7 +504,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   c->qkv = reinterpret_cast<u16*>(take(p.qkv));
   c->act = reinterpret_cast<u16*>(take(p.act));
   c->part = reinterpret_cast<float*>(take(p.part));
-  c->ws = take(p.ws);
+  c->ws = p.ws ? take(p.ws) : nullptr;
   // defined values wherever the tuning below reads (zero biases)
   e = hipMemset(c->base, 0, p.total());
   if (e != hipSuccess) {
@@ -518,7 +518,7 @@ int pi05_vision_create(const pi05_vision_dims* dims, pi05_vision_ctx** out) {
   bias.bias = true;
   GemmOpts fc2o = bias;
   fc2o.ld_k = kVIp;
-  const bool lib = M > kVLibRows;
+  const bool lib = p.ws != 0;
   bool ok = !lib || (lt_ok(hipblasLtCreate(&c->lt)) && make_plan(c->lt, M, kVQkvN, kVW, kVWorkspace, &c->g_qkv, &perr, bias) &&
                      make_plan(c->lt, M, kVW, kVW, kVWorkspace, &c->g_o, &perr, bias) && make_plan(c->lt, M, kVW, kVIp, kVWorkspace, &c->g_fc2, &perr, fc2o) &&
                      make_plan(c->lt, M, kVProj, kVW, kVWorkspace, &c->g_proj, &perr, bias));

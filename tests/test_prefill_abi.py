@@ -64,14 +64,25 @@ def test_device_bytes_covers_weights_and_activations(lib):
     need = 18 * (2560 * 2048 + 2048 * 2048 + 32768 * 2048 + 2048 * 16384) * 2  # packed bf16 weights (3.96 GB)
     need += 18 * 2 * 2048 * 4  # fp32 norm weights
     M = 968
-    need += M * (3 * 2048 + 2560 + 2048 + 32768 + 16384) * 2  # h, n, y, q|k|v, attention out, gate|up, GeGLU out
+    need += M * (3 * 2048 + 2560 + 2048 + 16384) * 2  # h, n, y, q|k|v, attention out, GeGLU out
     need += 992 * 8 * 256 * 2 + 2 * 992 * 256 * 2  # attention q fragments and K/V blocks (P padded to 992)
     need += 4 * 968 * 8 * (256 + 2) * 4  # 4 key splits (61 workgroups x 4 fill 244 CUs): fp32 partial O, max, sum
-    need += 4 * 968 * 2048 * 4  # down_proj split-K fp32 partials (4 slices)
+    need += 8 * 968 * 2048 * 4  # o_proj / down_proj split-K fp32 partials (up to 8 slices)
     got = _ext.prefix_device_bytes(d)
-    assert need <= got <= need + 80 * 2**20  # + GEMM workspace and small tables
+    assert need <= got <= need + 2 * 2**20  # + small tables; no library workspace up to 1024 rows
     d.batch = 2
     assert _ext.prefix_device_bytes(d) > got
+
+
+def test_device_bytes_hold_a_library_workspace_above_1024_rows_only(lib):
+    """One row more costs its activations (below 1 MiB); row 1025 the 64 MiB too, less one of the four key
+    splits' attention partials (8 heads x 258 floats a token: 8.1 MiB), which 129 tiles of tokens no longer take."""
+    d = _ext.prefix_default_dims()
+    sizes = []
+    for d.prefix_len in (1022, 1023, 1024, 1025, 1026):
+        sizes.append(_ext.prefix_device_bytes(d))
+    steps = [b - a for a, b in zip(sizes, sizes[1:])]
+    assert steps[2] >= 55 * 2**20 and all(0 < s < 2**20 for i, s in enumerate(steps) if i != 2), steps
 
 
 def test_null_handles_and_pointers(lib):

@@ -65,13 +65,16 @@ def test_device_bytes_covers_weights_and_activations(lib):
     Ip = 4352  # the MLP dim padded for 16-byte-aligned split-K slices of fc2
     need = 27 * (4 * W * W + I * W + W * Ip) * 2  # packed bf16 q|k|v, out, fc1, fc2 (0.8 GB)
     need += 27 * (3 * W + W + I + W + 4 * W) * 4  # fp32 biases and LayerNorm parameters
-    need += (W * 588 + W + S * W + 2 * W + P) * 4 + P * W * 2  # patch/position embeddings, post-LN, projector
+    need += (W * 592 + W + S * W + 2 * W + P) * 4 + P * W * 2  # patch (588 padded to 592) / position embeddings, post-LN, projector
     M = 3 * S
     need += M * (4 * W + 3 * W + Ip) * 2  # h, n, y, attention out, q|k|v, fc1 out
-    need += max(8 * M * W, 3 * M * Ip) * 4  # fp32 split-K partials: out_proj / fc2 (up to 8 slices), fc1 (up to 3)
-    need += M * (588 + W) * 4  # fp32 patches and patch-embedding output
+    need += 8 * M * W * 4  # fp32 split-K partials: out_proj / fc2 (up to 8 slices)
     got = _ext.vision_device_bytes(d)
-    assert need <= got <= need + 40 * 2**20  # + GEMM workspace
+    assert need <= got <= need + 2**20  # no library workspace up to 1024 rows (4 images)
+    d.n_images = 4
+    four = _ext.vision_device_bytes(d)
+    d.n_images = 5
+    assert 0 < four - got < 32 * 2**20 <= _ext.vision_device_bytes(d) - four - (four - got)
     d.n_images = 6
     assert _ext.vision_device_bytes(d) > got
 
