@@ -282,7 +282,7 @@ def bench_vision(args) -> int:
         "data": "synthetic (random-init SigLIP/projector weights N(0, 0.02), uniform [-1, 1] pixels, seeds 0/1)",
         "config": {"workload": f"SigLIP So400m/14 depth {L} + projector, {N} images of 224x224 (M = {N * 256})",
                    "n_images": N},
-        "roofline": {"kernel": "whole tower (HIP kernels)", "bound": "mfma",
+        "roofline": {"kernel": kernels_label("whole tower", ctx.products()), "bound": "mfma",
                      "achieved": round(tflops, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / BF16_PEAK_TFLOPS, 4), "traffic": None, "flops_per_call": flops},
         "cpu_baseline": cpu,
@@ -291,6 +291,12 @@ def bench_vision(args) -> int:
     ctx.close()
     torch.cuda.synchronize()
     return 0
+
+
+def kernels_label(what: str, products: dict) -> str:
+    """Which kernels a context's pass runs on, from what it chose per product when it was created."""
+    lib = [n for n, p in products.items() if p["library"]]
+    return f"{what} (HIP kernels; hipBLASLt: {', '.join(lib)})" if lib else f"{what} (HIP kernels)"
 
 
 def prefill_flops(depth: int, batch: int, prefix_len: int, skip_last: bool = True) -> int:
@@ -386,7 +392,7 @@ def bench_prefill(args) -> int:
         "data": "synthetic (random-init Gemma-2B weights N(0, 0.02), N(0,1) bf16 prefix embeddings, seed 0)",
         "config": {"workload": f"Gemma-2B prefix prefill, depth {L} (last layer K/V only), bs={B}, {P} tokens",
                    "batch": B, "prefix_len": P},
-        "roofline": {"kernel": "whole prefill (HIP kernels)", "bound": "mfma",
+        "roofline": {"kernel": kernels_label("whole prefill", ctx.products()), "bound": "mfma",
                      "achieved": round(tflops, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / BF16_PEAK_TFLOPS, 4), "traffic": None, "flops_per_prefill": flops},
         "cpu_baseline": cpu,

@@ -21,3 +21,10 @@ def test_more_than_one_gpu_is_refused_with_a_message():
 def test_flop_counts_match_the_published_phase_totals():
     assert round(bench.prefill_flops(18, 1, 968) / 1e9, 2) == 3756.15
     assert round(bench.vision_flops(27, 3) / 1e9, 2) == 660.53
+
+
+def test_label_names_the_products_that_the_library_runs():
+    own = dict.fromkeys(("qkv", "out_proj", "fc1"), {"library": False})
+    assert bench.kernels_label("whole tower", own) == "whole tower (HIP kernels)"
+    mixed = {**own, "qkv": {"library": True}, "out_proj": {"library": True}}
+    assert bench.kernels_label("whole tower", mixed) == "whole tower (HIP kernels; hipBLASLt: qkv, out_proj)"
