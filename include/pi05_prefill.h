@@ -112,7 +112,10 @@ int pi05_prefix_product(pi05_prefix_ctx* ctx, int which, int32_t* choice, float*
  * C[M, N] = A[M, K] . W[N, K]^T, bf16 operands with rows of lda / ldw elements, on tile `cfg`
  * (0 .. 7) with epilogue `epi` (0: bf16, optional fp32 bias[N]; 1: the same through GELU; 2: fp32
  * partial sums of `split` K splits, [split][M][ldc]; 3: GeGLU over W rows that alternate 16 gate and
- * 16 up rows, bf16 [M, N / 2]).  PI05_E_INVALID, and nothing enqueued, for a product that the tile does not take. */
+ * 16 up rows, bf16 [M, N / 2]).  epi + PI05_DEBUG_PRODUCT_CACHED: as for weights that stay in the cache behind the
+ * L2s (no lines fetched ahead), otherwise as for weights from HBM; the results are the same.  PI05_E_INVALID, and
+ * nothing enqueued, for a product that the tile does not take. */
+#define PI05_DEBUG_PRODUCT_CACHED 256
 int pi05_debug_product(int cfg, int epi, const void* a, const void* w, void* c, const float* bias, int M, int N, int K, int lda,
                        int ldw, int ldc, int split, void* stream);
 

@@ -870,7 +870,9 @@ int pi05_prefix_forward(pi05_prefix_ctx* c, const void* embeds, const uint8_t* p
 
 int pi05_debug_product(int cfg, int epi, const void* a, const void* w, void* c, const float* bias, int M, int N, int K, int lda, int ldw,
                        int ldc, int split, void* stream) {
-  const MmArgs args{static_cast<const u16*>(a), static_cast<const u16*>(w), c, bias, M, N, K, lda, ldw, ldc, split, 1};
+  const int cold = epi & PI05_DEBUG_PRODUCT_CACHED ? 0 : 1;
+  epi &= ~PI05_DEBUG_PRODUCT_CACHED;
+  const MmArgs args{static_cast<const u16*>(a), static_cast<const u16*>(w), c, bias, M, N, K, lda, ldw, ldc, split, cold};
   if (!a || !w || !c || epi < kMmBf16 || epi > kMmGeglu || !mm_fits(cfg, epi, args)) return fail(nullptr, PI05_E_INVALID, "the tile does not take this product");
   if (!mm_launch(cfg, epi, args, static_cast<hipStream_t>(stream))) return fail(nullptr, PI05_E_HIP, "product launch failed");
   return PI05_OK;

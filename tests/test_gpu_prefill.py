@@ -98,6 +98,26 @@ def test_prefill_parity_ragged_batch(layers3):
     _compare(ref, ks, vs, pad, "B2P77")
 
 
+@pytest.mark.parametrize("batch, plen, cut", [(1, 968, 900), (2, 550, 441), (3, 1100, 880)])
+def test_prefill_parity_of_large_prefixes(layers3, batch, plen, cut):
+    """968 rows, the headline's; 1100, where hipBLASLt is a candidate; 3300, beyond the rows that may be cut into 8 K
+    splits.  One full layer and the last one's K/V; the last sample is padded from `cut`."""
+    print(f"case prefill: depth 2, B={batch}, P={plen}, last sample padded from {cut}", flush=True)
+    torch.manual_seed(plen)
+    emb = O._bf(torch.randn(batch, plen, G.width))
+    pad = torch.ones(batch, plen, dtype=torch.bool)
+    pad[-1, cut:] = False
+    ref = PO.prefill(layers3[:2], G, emb, pad)
+    ctx, _keep = _context(2, batch, plen, layers3[:2])
+    choices = ctx.products()
+    print(choices, flush=True)
+    assert all((p["library_us"] > 0) == (batch * plen > 1024 and n != "gate_up") for n, p in choices.items())
+    assert choices["o_proj"]["splits"] <= 8 and choices["down_proj"]["splits"] <= (8 if batch * plen <= 3072 else 4)
+    ks, vs = _run(ctx, emb, pad, 2)
+    _compare(ref, ks, vs, pad, f"B{batch}P{plen}")
+    ctx.close()
+
+
 def test_kv_only_last_layer_matches_full_layer(layers3):
     print("case prefill: last layer K/V only vs full", flush=True)
     torch.manual_seed(2)
