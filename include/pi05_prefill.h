@@ -6,7 +6,7 @@
  * One context (`pi05_prefix_ctx`) owns the Gemma-2B layer weights (packed on refresh), the
  * activation buffers of one (batch, prefix_len) signature and its product plans.  Products, norms, RoPE
  * and the K/V write, the masked attention and GeGLU are hand-written gfx950 kernels; above 1024 rows
- * q|k|v, o_proj and down_proj run on hipBLASLt where it measured faster at creation.
+ * q|k|v, the last layer's k|v, o_proj and down_proj run on hipBLASLt where it measured faster at creation.
  *
  * Conventions are those of pi05_denoise.h: device pointers unless a name says `host`, bf16 as
  * raw bit patterns, 0 / negative PI05_E* codes with a message from pi05_prefix_last_error, every

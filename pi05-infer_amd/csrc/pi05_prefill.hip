@@ -8,8 +8,8 @@
 //   h += o . Wo^T; n = RMSNorm(h)            product (K splits) + rmsnorm_kernel (residual fused)
 //   a  = gelu_tanh(n . Wg^T) * (n . Wu^T)    product, N = 32768, GeGLU in its epilogue
 //   h += a . Wd^T; n = RMSNorm(h)            product (K splits) + rmsnorm_kernel
-// The products run on pi05_mm.h; from kLibRows rows on, q|k|v, o_proj and down_proj on hipBLASLt where it
-// measured faster when the context was created.
+// The products run on pi05_mm.h; above kLibRows rows q|k|v, the last layer's k|v, o_proj and down_proj on hipBLASLt
+// where it measured faster when the context was created.
 // The last layer computes only its K/V (patches/prefix_last_layer.py:84-112).  Every valid
 // token attends to every valid token of its sample (pi0_pytorch.py:236-250); positions are
 // cumsum(pad) - 1 (engine.py:776).
@@ -45,7 +45,10 @@ constexpr size_t kPLayerElems = kPOffD + (size_t)kPW * kPI;
 // partials grow with the rows: 4 splits hold 32 KiB a row)
 constexpr int kMaxSplits = 8, kSplitRows = 3072;
 int max_splits(int M) { return M <= kSplitRows ? kMaxSplits : 4; }
-// rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate
+// Rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate: down_proj is 22 to 34 % faster
+// here (968 rows: 63 us against 90), q|k|v and o_proj within 5 % either way (968: 16.0 / 15.3 and 13.9 / 14.2), the
+// last layer's k|v, once a pass, at most 2 us slower (512 rows: 8.6 / 6.8), and a context is there in 0.4 s instead of 1.0.
+// Above, the library gains (2848 rows: q|k|v 40 / 32, o_proj 36 / 27, but down_proj 146 / 171).
 constexpr int kLibRows = 1024;
 constexpr int kAttnMtPerWg = 8;  // attention m-tiles (16 query rows: 2 tokens x 8 heads) per workgroup
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt not waited for (gfx9 encoding:
@@ -528,7 +531,7 @@ struct pi05_prefix_ctx {
   unsigned embed_tag = 0, reported_tag = 0;
   void* ws = nullptr;
   hipblasLtHandle_t lt = nullptr;
-  // the products: on pi05_mm.h, or (from kLibRows rows, where it measured faster) on hipBLASLt
+  // the products: on pi05_mm.h, or (above kLibRows rows, where it measured faster) on hipBLASLt
   GemmPlan g_qkv, g_kv, g_o, g_d;
   MmPlan m_qkv, m_kv, m_o, m_gu, m_d;
   bool lib_qkv = false, lib_kv = false, lib_o = false, lib_d = false;

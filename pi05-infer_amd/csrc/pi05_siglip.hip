@@ -8,7 +8,7 @@
 //          h = bf16(h + a.W2^T + b2) ]         product (split-K when faster) + layernorm_kernel
 //                                              (the next LN1 / post_layernorm)
 //   out = (n.Wproj^T + bproj) * out_scale     product (+ scale_kernel)
-// The bf16 products run on pi05_mm.h; from kVLibRows rows on, q|k|v, out_proj, fc2 and the projector on
+// The bf16 products run on pi05_mm.h; above kVLibRows rows q|k|v, out_proj, fc2 and the projector on
 // hipBLASLt where it measured faster when the context was created.
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
@@ -44,7 +44,10 @@ constexpr size_t kVPOffBqkv = 0, kVPOffBo = kVQkvN, kVPOffB1 = kVPOffBo + kVW, k
                  kVPOffLn2b = kVPOffLn2w + kVW, kVLayerParams = kVPOffLn2b + kVW;
 constexpr size_t kVWorkspace = 32ull << 20;  // hipBLASLt's, where it is a candidate
 constexpr int kVMaxSplits = 8;  // K splits of out_proj and fc2 at most
-// rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate
+// Rows up to which the products run on pi05_mm.h alone, without a hipBLASLt candidate: a layer's products are faster
+// here in sum (us, here / library: 256 rows q|k|v 7.5 / 7.9, out_proj 5.5 / 6.7, fc2 8.7 / 14.0; 768 rows 11.8 / 11.4, 7.3 / 7.8,
+// 14.2 / 17.0; 1024 rows 14.5 / 13.2, 8.5 / 9.1, 17.6 / 21.5; the projector within 6 %), and a context is there in 0.15 s
+// instead of 0.6.  Above, the library gains (1280 rows: q|k|v 23 / 16; 6144 rows: 59 / 55 and out_proj 28 / 21).
 constexpr int kVLibRows = 1024;
 
 thread_local std::string g_vision_err;
@@ -409,7 +412,7 @@ struct pi05_vision_ctx {
         *part = nullptr;
   void* ws = nullptr;
   hipblasLtHandle_t lt = nullptr;
-  // the bf16 products: on pi05_mm.h, or (from kVLibRows rows, where it measured faster) on hipBLASLt
+  // the bf16 products: on pi05_mm.h, or (above kVLibRows rows, where it measured faster) on hipBLASLt
   GemmPlan g_qkv, g_o, g_fc2, g_proj;
   MmPlan m_qkv, m_o, m_fc1, m_fc2, m_proj;
   bool lib_qkv = false, lib_o = false, lib_fc2 = false, lib_proj = false;
