@@ -627,8 +627,8 @@ struct MmPlan {
 };
 
 // Operands for timing: normal values, as activations and weights are.  Zeros will not do: they switch little in the
-// matrix cores, so a large tile keeps a clock that it does not have in use (gate|up and its GeGLU, M = 1024: 88 us
-// on zeros, 102 on values of four exponents, 113 on normal ones; tiles up to 128 x 128: the same).  On zeros
+// matrix cores, so a large tile keeps a clock that it does not have in use (gate|up and its GeGLU, M = 1024: 87 us
+// on zeros, 102 on values of four exponents, 105 on normal ones; tiles up to 128 x 128: the same).  On zeros
 // down_proj at 968 rows took 192 x 256 (62 us on random values) in place of 256 x 192 (59).
 static __global__ __launch_bounds__(256) void mm_random_kernel(u16* p, size_t n, float std) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {

@@ -24,8 +24,8 @@ def test_projector_is_timed_as_it_runs(depth):
 
 def test_tiles_are_timed_on_values_that_switch_the_matrix_cores():
     """gate|up at 1024 rows (512 tiles of 256 x 256 on 256 CUs) runs faster on zeros than on normal values: the time
-    that the context chose its tile by is that of normal operands.  Measured 0.94 of it here, 0.79 when contexts
-    timed zeros; the line lies between the two."""
+    that the context chose its tile by must not be that of zeros.  Over the tile's time on zeros it measured 1.20
+    to 1.22 (105 / 86 us), and 1.00 to 1.02 when contexts timed zeros: the line lies between."""
     print("case prefill choices: depth 2, 1 x 1024", flush=True)
     d = _ext.prefix_default_dims()
     d.depth, d.batch, d.prefix_len = 2, 1, 1024
@@ -33,8 +33,7 @@ def test_tiles_are_timed_on_values_that_switch_the_matrix_cores():
     got = ctx.products()
     ctx.close()
     m, n, k = 1024, 32768, 2048
-    a = torch.randn(m, k, device="cuda").to(torch.bfloat16)
-    w = (torch.randn(2, n, k, device="cuda") * 0.02).to(torch.bfloat16)
+    a, w = torch.zeros(m, k, dtype=torch.bfloat16, device="cuda"), torch.zeros(2, n, k, dtype=torch.bfloat16, device="cuda")
     out = torch.empty(m, n // 2, dtype=torch.bfloat16, device="cuda")
     lib = _ext.load_prefix_library()
 
@@ -43,7 +42,7 @@ def test_tiles_are_timed_on_values_that_switch_the_matrix_cores():
                                       torch.cuda.current_stream().cuda_stream) == 0
 
     best, start, end = 1e9, torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    for _ in range(5):
+    for _ in range(6):
         once(1)
         start.record()
         for i in range(20):
@@ -51,5 +50,5 @@ def test_tiles_are_timed_on_values_that_switch_the_matrix_cores():
         end.record()
         end.synchronize()
         best = min(best, start.elapsed_time(end) / 20 * 1e3)
-    print(f"chosen by {got['gate_up']['us']:.1f} us, on random operands {best:.1f} us; {got}", flush=True)
-    assert got["gate_up"]["us"] >= 0.87 * best
+    print(f"chosen by {got['gate_up']['us']:.1f} us, on zeros {best:.1f} us; {got}", flush=True)
+    assert got["gate_up"]["us"] >= 1.11 * best
