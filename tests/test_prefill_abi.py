@@ -91,6 +91,7 @@ def test_null_handles_and_pointers(lib):
     assert lib.pi05_prefix_refresh_weights(None, None) == -1
     assert lib.pi05_prefix_embed_tokens(None, None, 1, None, 1, None, None) == -1
     assert lib.pi05_prefix_forward(None, None, None, None, None, 0, 256, None) == -1
+    assert lib.pi05_prefix_product(None, 0, None, None) == -1
     assert lib.pi05_prefix_create(None, None) == -1
     bad = _ext.prefix_default_dims()
     bad.head_dim = 64

@@ -85,6 +85,7 @@ def test_null_handles_and_pointers(lib):
     assert lib.pi05_vision_bind_heads(None, *([None] * 7)) == -1
     assert lib.pi05_vision_refresh_weights(None, None) == -1
     assert lib.pi05_vision_forward(None, None, None, None) == -1
+    assert lib.pi05_vision_product(None, 0, None, None) == -1
     assert lib.pi05_vision_create(None, None) == -1
     bad = _ext.vision_default_dims()
     bad.num_heads = 12
